@@ -38,6 +38,9 @@ inline void fill_geom(const ek_params& p, ek::Geom<T>& g, ek::Gas<T>& gas)
   g.idx = (T)(1.0 / p.dx);
   g.idy = (T)(1.0 / p.dy);
   g.idz = (T)(1.0 / p.dz);
+  g.rdx = 1.0 / p.dx;
+  g.rdy = 1.0 / p.dy;
+  g.rdz = 1.0 / p.dz;
   gas.gamma0 = (T)p.gamma0;
   gas.gamma6 = (T)p.gamma6;
   gas.gm1 = (T)(p.gamma0 - 1.0);

@@ -49,6 +49,7 @@ struct Geom {
   double dx, dy, dz;
   T tdx, tdy, tdz;    // dx.. in T
   T idx, idy, idz;    // 1/dx.. (exact when pow2)
+  double rdx, rdy, rdz; // 1/dx.. in FP64
   int pow2;
 };
 
@@ -287,7 +288,7 @@ __device__ __forceinline__ double cfl_term(const Gas<T>& gas, const T* u, const 
                                        geo.pow2 != 0);
   } else {
     const double d = fmax((double)u[ID], (double)gas.smallr);
-    const double id = 1.0 / d;
+    const double id = inv_of(d).y;
     const double ux = (double)u[IU] * id, uy = (double)u[IV] * id;
     double ek = ux * ux + uy * uy;
     double uz = 0.0;
@@ -297,10 +298,10 @@ __device__ __forceinline__ double cfl_term(const Gas<T>& gas, const T* u, const 
     }
     const double e = (double)u[IP] * id - 0.5 * ek;
     const double p = fmax((double)gas.gm1 * d * e, d * (double)gas.smallp);
-    const double c = sqrt((double)gas.gamma0 * p * id);
-    double s = (c + fabs(ux)) / geo.dx + (c + fabs(uy)) / geo.dy;
+    const double c = esqrt((double)gas.gamma0 * p * id);
+    double s = (c + fabs(ux)) * geo.rdx + (c + fabs(uy)) * geo.rdy;
     if constexpr (DIM == 3)
-      s += (c + fabs(uz)) / geo.dz;
+      s += (c + fabs(uz)) * geo.rdz;
     return s;
   }
 }

@@ -32,27 +32,29 @@ constexpr int NV = 8;
 
 // constoprim_mhd (src/muscl/MHDBaseFunctor2D.h:192-242), cIso = 0.
 template <class T>
-__host__ __device__ inline void constoprim(const Gas<T>& g, const T* u, T mx, T my, T mz, T* q)
+__device__ __forceinline__ void constoprim(const Gas<T>& g, const T* u, T mx, T my, T mz, T* q)
 {
   q[ID] = emax(u[ID], g.smallr);
-  q[IU] = u[IU] / q[ID];
-  q[IV] = u[IV] / q[ID];
-  q[IW] = u[IW] / q[ID];
+  const Inv<T> id = inv_of(q[ID]);
+  q[IU] = quot_any(u[IU], id);
+  q[IV] = quot_any(u[IV], id);
+  q[IW] = quot_any(u[IW], id);
   q[IA] = T(0.5) * (u[IA] + mx);
   q[IB] = T(0.5) * (u[IB] + my);
   q[IC] = T(0.5) * (u[IC] + mz);
   const T eken = T(0.5) * (q[IU] * q[IU] + q[IV] * q[IV] + q[IW] * q[IW]);
   const T emag = T(0.5) * (q[IA] * q[IA] + q[IB] * q[IB] + q[IC] * q[IC]);
-  T eint = (u[IP] - emag) / q[ID] - eken;
+  T eint = quot(u[IP] - emag, id) - eken;
   if constexpr (sizeof(T) == 4) {
     // FP32 state: p = (gamma-1)(E - rho v^2/2 - B^2/2) recovered in FP64 where more than 7
     // of the 24 mantissa bits cancel
-    if (eint < T(0.0078125) * (u[IP] / q[ID])) {
-      const double d = q[ID], ux = (double)u[IU] / d, uy = (double)u[IV] / d, uz = (double)u[IW] / d;
+    if (eint < T(0.0078125) * quot(u[IP], id)) {
+      const double rd = inv_of((double)q[ID]).y;
+      const double ux = (double)u[IU] * rd, uy = (double)u[IV] * rd, uz = (double)u[IW] * rd;
       const double bx = 0.5 * ((double)u[IA] + (double)mx), by = 0.5 * ((double)u[IB] + (double)my),
                    bz = 0.5 * ((double)u[IC] + (double)mz);
       const double em = 0.5 * (bx * bx + by * by + bz * bz);
-      eint = (T)(((double)u[IP] - em) / d - 0.5 * (ux * ux + uy * uy + uz * uz));
+      eint = (T)(((double)u[IP] - em) * rd - 0.5 * (ux * ux + uy * uy + uz * uz));
     }
   }
   q[IP] = emax(g.gm1 * q[ID] * eint, q[ID] * g.smallp);
@@ -60,32 +62,34 @@ __host__ __device__ inline void constoprim(const Gas<T>& g, const T* u, T mx, T 
 
 // find_speed_fast<dir> (src/shared/mhd_utils.h:89-117)
 template <class T, int DIR>
-__host__ __device__ inline T speed_fast(const Gas<T>& g, const T* q)
+__device__ __forceinline__ T speed_fast(const Gas<T>& g, const T* q)
 {
   const T d = q[ID], p = q[IP], a = q[IA], b = q[IB], c = q[IC];
   const T b2 = a * a + b * b + c * c;
-  const T c2 = g.gamma0 * p / d;
-  const T d2 = T(0.5) * (b2 / d + c2);
+  const Inv<T> id = inv_of(d);
+  const T c2 = quot(g.gamma0 * p, id);
+  const T d2 = T(0.5) * (quot(b2, id) + c2);
   const T n = DIR == 0 ? a : (DIR == 1 ? b : c);
-  return esqrt(d2 + esqrt(d2 * d2 - c2 * n * n / d));
+  return esqrt(d2 + esqrt(d2 * d2 - quot(c2 * n * n, id)));
 }
 
 // find_speed_info<TWO_D> (mhd_utils.h:319-366) folded into ComputeDtFunctor2D_MHD
 // (src/muscl/MHDRunFunctors2D.h:36-74): vx/dx + vy/dy.
 template <class T>
-__host__ __device__ inline T cell_inv_dt(const Gas<T>& g, const T* q, T dx, T dy, T idx, T idy, bool pow2)
+__device__ __forceinline__ T cell_inv_dt(const Gas<T>& g, const T* q, T dx, T dy, T idx, T idy, bool pow2)
 {
   const T d = q[ID], p = q[IP], a = q[IA], b = q[IB], c = q[IC];
   const T b2 = a * a + b * b + c * c;
-  const T c2 = g.gamma0 * p / d;
-  const T d2 = T(0.5) * (b2 / d + c2);
-  const T cfx = esqrt(d2 + esqrt(d2 * d2 - c2 * a * a / d));
+  const Inv<T> id = inv_of(d);
+  const T c2 = quot(g.gamma0 * p, id);
+  const T d2 = T(0.5) * (quot(b2, id) + c2);
+  const T cfx = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * a * a, id)));
   const T vx = cfx + eabs(q[IU]);
-  const T cfy = esqrt(d2 + esqrt(d2 * d2 - c2 * b * b / d));
+  const T cfy = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * b * b, id)));
   const T vy = cfy + eabs(q[IV]);
   if (pow2)
     return vx * idx + vy * idy;
-  return vx / dx + vy / dy;
+  return quot(vx, inv_with(dx, idx)) + quot(vy, inv_with(dy, idy));
 }
 
 // CFL term of an FP32 MHD cell, widened to FP64 so that the dt reduction always runs in
@@ -94,10 +98,10 @@ __host__ __device__ inline T cell_inv_dt(const Gas<T>& g, const T* q, T dx, T dy
 // where the reference's expressions have eight (2D) or ten (3D).
 template <int DIM>
 __device__ __forceinline__ double mhd_cfl_widened(const Gas<float>& gas, const float* u, double mx, double my,
-                                                  double mz, double dx, double dy, double dz)
+                                                  double mz, double rdx, double rdy, double rdz)
 {
   const double d = fmax((double)u[ID], (double)gas.smallr);
-  const double id = 1.0 / d;
+  const double id = inv_of(d).y;
   const double ux = (double)u[IU] * id, uy = (double)u[IV] * id, uz = (double)u[IW] * id;
   const double a = 0.5 * ((double)u[IA] + mx), b = 0.5 * ((double)u[IB] + my), c = 0.5 * ((double)u[IC] + mz);
   const double eken = 0.5 * (ux * ux + uy * uy + uz * uz);
@@ -106,12 +110,12 @@ __device__ __forceinline__ double mhd_cfl_widened(const Gas<float>& gas, const f
   const double p = fmax((double)gas.gm1 * d * eint, d * (double)gas.smallp);
   const double c2 = (double)gas.gamma0 * p * id;
   const double d2 = 0.5 * (b2 * id + c2);
-  const double vx = sqrt(d2 + sqrt(d2 * d2 - c2 * a * a * id)) + fabs(ux);
-  const double vy = sqrt(d2 + sqrt(d2 * d2 - c2 * b * b * id)) + fabs(uy);
-  double s = vx / dx + vy / dy;
+  const double vx = esqrt(d2 + esqrt(d2 * d2 - c2 * a * a * id)) + fabs(ux);
+  const double vy = esqrt(d2 + esqrt(d2 * d2 - c2 * b * b * id)) + fabs(uy);
+  double s = vx * rdx + vy * rdy;
   if constexpr (DIM == 3) {
-    const double vz = sqrt(d2 + sqrt(d2 * d2 - c2 * c * c * id)) + fabs(uz);
-    s += vz / dz;
+    const double vz = esqrt(d2 + esqrt(d2 * d2 - c2 * c * c * id)) + fabs(uz);
+    s += vz * rdz;
   }
   return s;
 }
@@ -126,13 +130,13 @@ __device__ __forceinline__ double mhd_cfl_term(const Gas<T>& gas, const T* u, T 
     constoprim<T>(gas, u, mx, my, T(0), q);
     return cell_inv_dt<T>(gas, q, geo.tdx, geo.tdy, geo.idx, geo.idy, geo.pow2 != 0);
   } else {
-    return mhd_cfl_widened<2>(gas, u, (double)mx, (double)my, 0.0, geo.dx, geo.dy, 1.0);
+    return mhd_cfl_widened<2>(gas, u, (double)mx, (double)my, 0.0, geo.rdx, geo.rdy, 1.0);
   }
 }
 
 // find_mhd_flux (mhd_utils.h:173-231)
 template <class T>
-__host__ __device__ inline void mhd_flux(const Gas<T>& g, const T* q, T* cv, T* ff)
+__device__ __forceinline__ void mhd_flux(const Gas<T>& g, const T* q, T* cv, T* ff)
 {
   const T d = q[ID], p = q[IP], u = q[IU], v = q[IV], w = q[IW], a = q[IA], b = q[IB], c = q[IC];
   const T ecin = T(0.5) * (u * u + v * v + w * w) * d;
@@ -159,7 +163,7 @@ __host__ __device__ inline void mhd_flux(const Gas<T>& g, const T* q, T* cv, T* 
 
 // riemann_hll, MHD (src/shared/RiemannSolvers_MHD.h:24-64)
 template <class T>
-__host__ __device__ inline void hll(const Gas<T>& g, T* ql, T* qr, T* flux)
+__device__ __forceinline__ void hll(const Gas<T>& g, T* ql, T* qr, T* flux)
 {
   const T bx = T(0.5) * (ql[IA] + qr[IA]);
   ql[IA] = bx;
@@ -170,14 +174,15 @@ __host__ __device__ inline void hll(const Gas<T>& g, T* ql, T* qr, T* flux)
   const T cfl = speed_fast<T, 0>(g, ql), cfr = speed_fast<T, 0>(g, qr);
   const T sl = emin(emin(ql[IU], qr[IU]) - emax(cfl, cfr), T(0));
   const T sr = emax(emax(ql[IU], qr[IU]) + emax(cfl, cfr), T(0));
+  const Inv<T> iw = inv_of(sr - sl);
 #pragma unroll
   for (int n = 0; n < NV; n++)
-    flux[n] = (sr * fl[n] - sl * fr[n] + sr * sl * (ur[n] - ul[n])) / (sr - sl);
+    flux[n] = quot_any(sr * fl[n] - sl * fr[n] + sr * sl * (ur[n] - ul[n]), iw);
 }
 
 // riemann_llf, MHD (RiemannSolvers_MHD.h:78-110)
 template <class T>
-__host__ __device__ inline void llf(const Gas<T>& g, T* ql, T* qr, T* flux)
+__device__ __forceinline__ void llf(const Gas<T>& g, T* ql, T* qr, T* flux)
 {
   const T bx = T(0.5) * (ql[IA] + qr[IA]);
   ql[IA] = bx;
@@ -198,7 +203,7 @@ __host__ __device__ inline void llf(const Gas<T>& g, T* ql, T* qr, T* flux)
 
 // riemann_hlld (RiemannSolvers_MHD.h:130-364)
 template <class T>
-__host__ __device__ inline void hlld(const Gas<T>& g, const T* qleft, const T* qright, T* flux)
+__device__ __forceinline__ void hlld(const Gas<T>& g, const T* qleft, const T* qright, T* flux)
 {
   const T a = T(0.5) * (qleft[IA] + qright[IA]);
   const T sgnm = (a >= T(0)) ? T(1) : T(-1);
@@ -226,50 +231,62 @@ __host__ __device__ inline void hlld(const Gas<T>& g, const T* qleft, const T* q
   const T sr = emax(ul, ur) + emax(cfastl, cfastr);
   const T rcl = rl * (ul - sl);
   const T rcr = rr * (sr - ur);
-  const T ustar = (rcr * ur + rcl * ul + (ptotl - ptotr)) / (rcr + rcl);
-  const T ptotstar = (rcr * ptotl + rcl * ptotr + rcl * rcr * (ul - ur)) / (rcr + rcl);
+  const Inv<T> irc = inv_of(rcr + plain(rcl)); // FP32: only rcr's product fuses into the sum
+  const T ustar = quot_any(rcr * ur + rcl * ul + (ptotl - ptotr), irc);
+  const T ptotstar = quot(rcr * ptotl + rcl * ptotr + rcl * rcr * (ul - ur), irc);
+  const Inv<T> iaa = inv_of(a * a);
   // left star region
-  const T rstarl = rl * (sl - ul) / (sl - ustar);
+  const Inv<T> isl = inv_of(sl - ustar);
+  const T rstarl = quot(rl * (sl - ul), isl);
   T estar = rl * (sl - ul) * (sl - ustar) - a * a;
   const T el = rl * (sl - ul) * (sl - ul) - a * a;
   T vstarl, wstarl, bstarl, cstarl;
-  if (a * a > T(0) && eabs(estar / (a * a) - T(1)) <= T(1e-8)) {
+  if (a * a > T(0) && eabs(quot(estar, iaa) - T(1)) <= T(1e-8)) {
     vstarl = vl; bstarl = bl; wstarl = wl; cstarl = cl;
   } else {
-    vstarl = vl - a * bl * (ustar - ul) / estar;
-    bstarl = bl * el / estar;
-    wstarl = wl - a * cl * (ustar - ul) / estar;
-    cstarl = cl * el / estar;
+    const Inv<T> ie = inv_of(estar);
+    vstarl = vl - quot_any(a * bl * (ustar - ul), ie);
+    bstarl = quot_any(bl * el, ie);
+    wstarl = wl - quot_any(a * cl * (ustar - ul), ie);
+    cstarl = quot_any(cl * el, ie);
   }
   const T vdotbstarl = ustar * a + vstarl * bstarl + wstarl * cstarl;
-  const T etotstarl = ((sl - ul) * etotl - ptotl * ul + ptotstar * ustar + a * (vdotbl - vdotbstarl)) / (sl - ustar);
-  const T sqrrstarl = esqrt(rstarl);
-  const T calfvenl = eabs(a) / sqrrstarl;
+  const T etotstarl =
+      quot((sl - ul) * etotl - ptotl * ul + ptotstar * ustar + a * (vdotbl - vdotbstarl), isl);
+  const RootInv<T> rootl = sqrt_inv(rstarl);
+  const T sqrrstarl = rootl.s;
+  const T calfvenl = quot(eabs(a), rootl.inv);
   const T sal = ustar - calfvenl;
   // right star region
-  const T rstarr = rr * (sr - ur) / (sr - ustar);
+  const Inv<T> isr = inv_of(sr - ustar);
+  const T rstarr = quot(rr * (sr - ur), isr);
   estar = rr * (sr - ur) * (sr - ustar) - a * a;
   const T er = rr * (sr - ur) * (sr - ur) - a * a;
   T vstarr, wstarr, bstarr, cstarr;
-  if (a * a > T(0) && eabs(estar / (a * a) - T(1)) <= T(1e-8)) {
+  if (a * a > T(0) && eabs(quot(estar, iaa) - T(1)) <= T(1e-8)) {
     vstarr = vr; bstarr = br; wstarr = wr; cstarr = cr;
   } else {
-    vstarr = vr - a * br * (ustar - ur) / estar;
-    bstarr = br * er / estar;
-    wstarr = wr - a * cr * (ustar - ur) / estar;
-    cstarr = cr * er / estar;
+    const Inv<T> ie = inv_of(estar);
+    vstarr = vr - quot_any(a * br * (ustar - ur), ie);
+    bstarr = quot_any(br * er, ie);
+    wstarr = wr - quot_any(a * cr * (ustar - ur), ie);
+    cstarr = quot_any(cr * er, ie);
   }
   const T vdotbstarr = ustar * a + vstarr * bstarr + wstarr * cstarr;
-  const T etotstarr = ((sr - ur) * etotr - ptotr * ur + ptotstar * ustar + a * (vdotbr - vdotbstarr)) / (sr - ustar);
-  const T sqrrstarr = esqrt(rstarr);
-  const T calfvenr = eabs(a) / sqrrstarr;
+  const T etotstarr =
+      quot((sr - ur) * etotr - ptotr * ur + ptotstar * ustar + a * (vdotbr - vdotbstarr), isr);
+  const RootInv<T> rootr = sqrt_inv(rstarr);
+  const T sqrrstarr = rootr.s;
+  const T calfvenr = quot(eabs(a), rootr.inv);
   const T sar = ustar + calfvenr;
   // double star region
-  const T den = sqrrstarl + sqrrstarr;
-  const T vstarstar = (sqrrstarl * vstarl + sqrrstarr * vstarr + sgnm * (bstarr - bstarl)) / den;
-  const T wstarstar = (sqrrstarl * wstarl + sqrrstarr * wstarr + sgnm * (cstarr - cstarl)) / den;
-  const T bstarstar = (sqrrstarl * bstarr + sqrrstarr * bstarl + sgnm * sqrrstarl * sqrrstarr * (vstarr - vstarl)) / den;
-  const T cstarstar = (sqrrstarl * cstarr + sqrrstarr * cstarl + sgnm * sqrrstarl * sqrrstarr * (wstarr - wstarl)) / den;
+  const Inv<T> iden = inv_of(sqrrstarl + sqrrstarr);
+  const T vstarstar = quot_any(sqrrstarl * vstarl + sqrrstarr * vstarr + sgnm * (bstarr - bstarl), iden);
+  const T wstarstar = quot_any(sqrrstarl * wstarl + sqrrstarr * wstarr + sgnm * (cstarr - cstarl), iden);
+  const T bstarstar =
+      quot_any(sqrrstarl * bstarr + sqrrstarr * bstarl + sgnm * sqrrstarl * sqrrstarr * (vstarr - vstarl), iden);
+  const T cstarstar =
+      quot_any(sqrrstarl * cstarr + sqrrstarr * cstarl + sgnm * sqrrstarl * sqrrstarr * (wstarr - wstarl), iden);
   const T vdotbstarstar = ustar * a + vstarstar * bstarstar + wstarstar * cstarstar;
   const T etotstarstarl = etotstarl - sgnm * sqrrstarl * (vdotbstarl - vdotbstarstar);
   const T etotstarstarr = etotstarr + sgnm * sqrrstarr * (vdotbstarr - vdotbstarstar);
@@ -303,7 +320,7 @@ __host__ __device__ inline void hlld(const Gas<T>& g, const T* qleft, const T* q
 
 // riemann_mhd dispatch (RiemannSolvers_MHD.h:369-389)
 template <class T, int RS>
-__host__ __device__ inline void riemann(const Gas<T>& g, T* ql, T* qr, T* f)
+__device__ __forceinline__ void riemann(const Gas<T>& g, T* ql, T* qr, T* f)
 {
   if constexpr (RS == RS_HLLD)
     hlld<T>(g, ql, qr, f);
@@ -315,7 +332,7 @@ __host__ __device__ inline void riemann(const Gas<T>& g, T* ql, T* qr, T* f)
 
 // FMAX4 / FMIN4 / FMAX5 (src/shared/mhd_utils.h:17-60): sequential strict compares
 template <class T>
-__host__ __device__ inline T fmax4(T a0, T a1, T a2, T a3)
+__device__ __forceinline__ T fmax4(T a0, T a1, T a2, T a3)
 {
   T r = a0;
   r = (a1 > r) ? a1 : r;
@@ -324,7 +341,7 @@ __host__ __device__ inline T fmax4(T a0, T a1, T a2, T a3)
   return r;
 }
 template <class T>
-__host__ __device__ inline T fmin4(T a0, T a1, T a2, T a3)
+__device__ __forceinline__ T fmin4(T a0, T a1, T a2, T a3)
 {
   T r = a0;
   r = (a1 < r) ? a1 : r;
@@ -333,7 +350,7 @@ __host__ __device__ inline T fmin4(T a0, T a1, T a2, T a3)
   return r;
 }
 template <class T>
-__host__ __device__ inline T fmax5(T a0, T a1, T a2, T a3, T a4)
+__device__ __forceinline__ T fmax5(T a0, T a1, T a2, T a3, T a4)
 {
   T r = a0;
   r = (a1 > r) ? a1 : r;
@@ -349,28 +366,23 @@ struct Edge {
   T r, p, u, v, a, b, c;
 };
 
+// find_speed_fast along both directions of the edge plane (src/shared/mhd_utils.h:89-117)
 template <class T>
-__host__ __device__ inline T fast_x(const Gas<T>& g, const Edge<T>& s)
+__device__ __forceinline__ void fast_xy(const Gas<T>& g, const Edge<T>& s, T& fx, T& fy)
 {
   const T b2 = s.a * s.a + s.b * s.b + s.c * s.c;
-  const T c2 = g.gamma0 * s.p / s.r;
-  const T d2 = T(0.5) * (b2 / s.r + c2);
-  return esqrt(d2 + esqrt(d2 * d2 - c2 * s.a * s.a / s.r));
-}
-template <class T>
-__host__ __device__ inline T fast_y(const Gas<T>& g, const Edge<T>& s)
-{
-  const T b2 = s.a * s.a + s.b * s.b + s.c * s.c;
-  const T c2 = g.gamma0 * s.p / s.r;
-  const T d2 = T(0.5) * (b2 / s.r + c2);
-  return esqrt(d2 + esqrt(d2 * d2 - c2 * s.b * s.b / s.r));
+  const Inv<T> ir = inv_of(s.r);
+  const T c2 = quot(g.gamma0 * s.p, ir);
+  const T d2 = T(0.5) * (quot(b2, ir) + c2);
+  fx = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * s.a * s.a, ir)));
+  fy = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * s.b * s.b, ir)));
 }
 
 // compute_emf<EMFZ> + mag_riemann2d_hlld (RiemannSolvers_MHD.h:395-627, 648-871). The
 // edge states arrive as the trace produced them (qRT, qRB, qLT, qLB); the solver's
 // LL/RL/LR/RR states are RT/LT/RB/LB with the transverse face fields averaged.
 template <class T>
-__host__ __device__ inline T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edge<T>& RB, const Edge<T>& LT,
+__device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edge<T>& RB, const Edge<T>& LT,
                                    const Edge<T>& LB)
 {
   Edge<T> LL = RT, RL = LT, LR = RB, RR = LB;
@@ -388,89 +400,99 @@ __host__ __device__ inline T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
   const T rLR = LR.r, uLR = LR.u, vLR = LR.v, aLR = LR.a, bLR = LR.b, cLR = LR.c, pLR = LR.p;
   const T rRL = RL.r, uRL = RL.u, vRL = RL.v, aRL = RL.a, bRL = RL.b, cRL = RL.c, pRL = RL.p;
   const T rRR = RR.r, uRR = RR.u, vRR = RR.v, aRR = RR.a, bRR = RR.b, cRR = RR.c, pRR = RR.p;
-  const T SL = fmin4(uLL, uLR, uRL, uRR) - fmax4(fast_x(g, LL), fast_x(g, LR), fast_x(g, RL), fast_x(g, RR));
-  const T SR = fmax4(uLL, uLR, uRL, uRR) + fmax4(fast_x(g, LL), fast_x(g, LR), fast_x(g, RL), fast_x(g, RR));
-  const T SB = fmin4(vLL, vLR, vRL, vRR) - fmax4(fast_y(g, LL), fast_y(g, LR), fast_y(g, RL), fast_y(g, RR));
-  const T ST = fmax4(vLL, vLR, vRL, vRR) + fmax4(fast_y(g, LL), fast_y(g, LR), fast_y(g, RL), fast_y(g, RR));
+  T fxLL, fxLR, fxRL, fxRR, fyLL, fyLR, fyRL, fyRR;
+  fast_xy(g, LL, fxLL, fyLL);
+  fast_xy(g, LR, fxLR, fyLR);
+  fast_xy(g, RL, fxRL, fyRL);
+  fast_xy(g, RR, fxRR, fyRR);
+  const T fx = fmax4(fxLL, fxLR, fxRL, fxRR), fy = fmax4(fyLL, fyLR, fyRL, fyRR);
+  const T SL = fmin4(uLL, uLR, uRL, uRR) - fx;
+  const T SR = fmax4(uLL, uLR, uRL, uRR) + fx;
+  const T SB = fmin4(vLL, vLR, vRL, vRR) - fy;
+  const T ST = fmax4(vLL, vLR, vRL, vRR) + fy;
   const T PtotLL = pLL + T(0.5) * (aLL * aLL + bLL * bLL + cLL * cLL);
   const T PtotLR = pLR + T(0.5) * (aLR * aLR + bLR * bLR + cLR * cLR);
   const T PtotRL = pRL + T(0.5) * (aRL * aRL + bRL * bRL + cRL * cRL);
   const T PtotRR = pRR + T(0.5) * (aRR * aRR + bRR * bRR + cRR * cRR);
   const T rcLLx = rLL * (uLL - SL), rcRLx = rRL * (SR - uRL), rcLRx = rLR * (uLR - SL), rcRRx = rRR * (SR - uRR);
   const T rcLLy = rLL * (vLL - SB), rcLRy = rLR * (ST - vLR), rcRLy = rRL * (vRL - SB), rcRRy = rRR * (ST - vRR);
-  const T ustar = (rcLLx * uLL + rcLRx * uLR + rcRLx * uRL + rcRRx * uRR + (PtotLL - PtotRL + PtotLR - PtotRR)) /
-                  (rcLLx + rcLRx + rcRLx + rcRRx);
-  const T vstar = (rcLLy * vLL + rcLRy * vLR + rcRLy * vRL + rcRRy * vRR + (PtotLL - PtotLR + PtotRL - PtotRR)) /
-                  (rcLLy + rcLRy + rcRLy + rcRRy);
-  const T rstarLLx = rLL * (SL - uLL) / (SL - ustar);
-  const T BstarLL = bLL * (SL - uLL) / (SL - ustar);
-  const T rstarLLy = rLL * (SB - vLL) / (SB - vstar);
-  const T AstarLL = aLL * (SB - vLL) / (SB - vstar);
-  const T rstarLL = rLL * (SL - uLL) / (SL - ustar) * (SB - vLL) / (SB - vstar);
+  const T ustar =
+      quot_any(rcLLx * uLL + rcLRx * uLR + rcRLx * uRL + rcRRx * uRR + (PtotLL - PtotRL + PtotLR - PtotRR),
+               inv_of(rcLLx + rcLRx + rcRLx + rcRRx));
+  const T vstar =
+      quot_any(rcLLy * vLL + rcLRy * vLR + rcRLy * vRL + rcRRy * vRR + (PtotLL - PtotLR + PtotRL - PtotRR),
+               inv_of(rcLLy + rcLRy + rcRLy + rcRRy));
+  const Inv<T> iL = inv_of(SL - ustar), iR = inv_of(SR - ustar), iB = inv_of(SB - vstar), iT = inv_of(ST - vstar);
+  const T rstarLLx = quot(rLL * (SL - uLL), iL);
+  const T BstarLL = quot_any(bLL * (SL - uLL), iL);
+  const T rstarLLy = quot(rLL * (SB - vLL), iB);
+  const T AstarLL = quot_any(aLL * (SB - vLL), iB);
+  const T rstarLL = quot(rstarLLx * (SB - vLL), iB);
   const T EstarLLx = ustar * BstarLL - vLL * aLL;
   const T EstarLLy = uLL * bLL - vstar * AstarLL;
   const T EstarLL = ustar * BstarLL - vstar * AstarLL;
-  const T rstarLRx = rLR * (SL - uLR) / (SL - ustar);
-  const T BstarLR = bLR * (SL - uLR) / (SL - ustar);
-  const T rstarLRy = rLR * (ST - vLR) / (ST - vstar);
-  const T AstarLR = aLR * (ST - vLR) / (ST - vstar);
-  const T rstarLR = rLR * (SL - uLR) / (SL - ustar) * (ST - vLR) / (ST - vstar);
+  const T rstarLRx = quot(rLR * (SL - uLR), iL);
+  const T BstarLR = quot_any(bLR * (SL - uLR), iL);
+  const T rstarLRy = quot(rLR * (ST - vLR), iT);
+  const T AstarLR = quot_any(aLR * (ST - vLR), iT);
+  const T rstarLR = quot(rstarLRx * (ST - vLR), iT);
   const T EstarLRx = ustar * BstarLR - vLR * aLR;
   const T EstarLRy = uLR * bLR - vstar * AstarLR;
   const T EstarLR = ustar * BstarLR - vstar * AstarLR;
-  const T rstarRLx = rRL * (SR - uRL) / (SR - ustar);
-  const T BstarRL = bRL * (SR - uRL) / (SR - ustar);
-  const T rstarRLy = rRL * (SB - vRL) / (SB - vstar);
-  const T AstarRL = aRL * (SB - vRL) / (SB - vstar);
-  const T rstarRL = rRL * (SR - uRL) / (SR - ustar) * (SB - vRL) / (SB - vstar);
+  const T rstarRLx = quot(rRL * (SR - uRL), iR);
+  const T BstarRL = quot_any(bRL * (SR - uRL), iR);
+  const T rstarRLy = quot(rRL * (SB - vRL), iB);
+  const T AstarRL = quot_any(aRL * (SB - vRL), iB);
+  const T rstarRL = quot(rstarRLx * (SB - vRL), iB);
   const T EstarRLx = ustar * BstarRL - vRL * aRL;
   const T EstarRLy = uRL * bRL - vstar * AstarRL;
   const T EstarRL = ustar * BstarRL - vstar * AstarRL;
-  const T rstarRRx = rRR * (SR - uRR) / (SR - ustar);
-  const T BstarRR = bRR * (SR - uRR) / (SR - ustar);
-  const T rstarRRy = rRR * (ST - vRR) / (ST - vstar);
-  const T AstarRR = aRR * (ST - vRR) / (ST - vstar);
-  const T rstarRR = rRR * (SR - uRR) / (SR - ustar) * (ST - vRR) / (ST - vstar);
+  const T rstarRRx = quot(rRR * (SR - uRR), iR);
+  const T BstarRR = quot_any(bRR * (SR - uRR), iR);
+  const T rstarRRy = quot(rRR * (ST - vRR), iT);
+  const T AstarRR = quot_any(aRR * (ST - vRR), iT);
+  const T rstarRR = quot(rstarRRx * (ST - vRR), iT);
   const T EstarRRx = ustar * BstarRR - vRR * aRR;
   const T EstarRRy = uRR * bRR - vstar * AstarRR;
   const T EstarRR = ustar * BstarRR - vstar * AstarRR;
-  const T calfvenL = fmax5(eabs(aLR) / esqrt(rstarLRx), eabs(AstarLR) / esqrt(rstarLR), eabs(aLL) / esqrt(rstarLLx),
-                           eabs(AstarLL) / esqrt(rstarLL), g.smallc);
-  const T calfvenR = fmax5(eabs(aRR) / esqrt(rstarRRx), eabs(AstarRR) / esqrt(rstarRR), eabs(aRL) / esqrt(rstarRLx),
-                           eabs(AstarRL) / esqrt(rstarRL), g.smallc);
-  const T calfvenB = fmax5(eabs(bLL) / esqrt(rstarLLy), eabs(BstarLL) / esqrt(rstarLL), eabs(bRL) / esqrt(rstarRLy),
-                           eabs(BstarRL) / esqrt(rstarRL), g.smallc);
-  const T calfvenT = fmax5(eabs(bLR) / esqrt(rstarLRy), eabs(BstarLR) / esqrt(rstarLR), eabs(bRR) / esqrt(rstarRRy),
-                           eabs(BstarRR) / esqrt(rstarRR), g.smallc);
+  const Inv<T> qLL = sqrt_inv(rstarLL).inv, qLR = sqrt_inv(rstarLR).inv;
+  const Inv<T> qRL = sqrt_inv(rstarRL).inv, qRR = sqrt_inv(rstarRR).inv;
+  const T calfvenL = fmax5(quot(eabs(aLR), sqrt_inv(rstarLRx).inv), quot(eabs(AstarLR), qLR),
+                           quot(eabs(aLL), sqrt_inv(rstarLLx).inv), quot(eabs(AstarLL), qLL), g.smallc);
+  const T calfvenR = fmax5(quot(eabs(aRR), sqrt_inv(rstarRRx).inv), quot(eabs(AstarRR), qRR),
+                           quot(eabs(aRL), sqrt_inv(rstarRLx).inv), quot(eabs(AstarRL), qRL), g.smallc);
+  const T calfvenB = fmax5(quot(eabs(bLL), sqrt_inv(rstarLLy).inv), quot(eabs(BstarLL), qLL),
+                           quot(eabs(bRL), sqrt_inv(rstarRLy).inv), quot(eabs(BstarRL), qRL), g.smallc);
+  const T calfvenT = fmax5(quot(eabs(bLR), sqrt_inv(rstarLRy).inv), quot(eabs(BstarLR), qLR),
+                           quot(eabs(bRR), sqrt_inv(rstarRRy).inv), quot(eabs(BstarRR), qRR), g.smallc);
   const T SAL = emin(ustar - calfvenL, T(0));
   const T SAR = emax(ustar + calfvenR, T(0));
   const T SAB = emin(vstar - calfvenB, T(0));
   const T SAT = emax(vstar + calfvenT, T(0));
-  const T AstarT = (SAR * AstarRR - SAL * AstarLR) / (SAR - SAL);
-  const T AstarB = (SAR * AstarRL - SAL * AstarLL) / (SAR - SAL);
-  const T BstarR = (SAT * BstarRR - SAB * BstarRL) / (SAT - SAB);
-  const T BstarL = (SAT * BstarLR - SAB * BstarLL) / (SAT - SAB);
-  // branch selectors as 0/1 integers; the reference blends all five candidates with them,
+  const Inv<T> iw = inv_of(SAR - SAL), ih = inv_of(SAT - SAB);
+  const T AstarT = quot_any(SAR * AstarRR - SAL * AstarLR, iw);
+  const T AstarB = quot_any(SAR * AstarRL - SAL * AstarLL, iw);
+  const T BstarR = quot_any(SAT * BstarRR - SAB * BstarRL, ih);
+  const T BstarL = quot_any(SAT * BstarLR - SAB * BstarLL, ih);
+  // branch selectors as 0/1 factors; the reference blends all five candidates with them,
   // so a non-finite unused candidate still reaches the result (0 * inf = NaN) -- kept.
-  const int SB_pos = (int)(T(1) + ecopysign(T(1), SB)) / 2, SB_neg = 1 - SB_pos;
-  const int ST_pos = (int)(T(1) + ecopysign(T(1), ST)) / 2, ST_neg = 1 - ST_pos;
-  const int SL_pos = (int)(T(1) + ecopysign(T(1), SL)) / 2, SL_neg = 1 - SL_pos;
-  const int SR_pos = (int)(T(1) + ecopysign(T(1), SR)) / 2, SR_neg = 1 - SR_pos;
+  const bool Bp = !signbit_of(SB), Tp = !signbit_of(ST), Lp = !signbit_of(SL), Rp = !signbit_of(SR);
+  auto on = [](bool b) -> T { return b ? T(1) : T(0); };
   T E = T(0), tmpE;
-  tmpE = (SAL * SAB * EstarRR - SAL * SAT * EstarRL - SAR * SAB * EstarLR + SAR * SAT * EstarLL) / (SAR - SAL) /
-             (SAT - SAB) -
-         SAT * SAB / (SAT - SAB) * (AstarT - AstarB) + SAR * SAL / (SAR - SAL) * (BstarR - BstarL);
-  E += T(SB_neg * ST_pos * SL_neg * SR_pos) * tmpE;
-  tmpE = (SAR * EstarLLx - SAL * EstarRLx + SAR * SAL * (bRL - bLL)) / (SAR - SAL);
-  tmpE = T(SL_pos) * ELL + T(SL_neg * SR_neg) * ERL + T(SL_neg * SR_pos) * tmpE;
-  E += T(SB_pos) * tmpE;
-  tmpE = (SAR * EstarLRx - SAL * EstarRRx + SAR * SAL * (bRR - bLR)) / (SAR - SAL);
-  tmpE = T(SL_pos) * ELR + T(SL_neg * SR_neg) * ERR + T(SL_neg * SR_pos) * tmpE;
-  E += T(SB_neg * ST_neg) * tmpE;
-  tmpE = (SAT * EstarLLy - SAB * EstarLRy - SAT * SAB * (aLR - aLL)) / (SAT - SAB);
-  E += T(SB_neg * ST_pos * SL_pos) * tmpE;
-  tmpE = (SAT * EstarRLy - SAB * EstarRRy - SAT * SAB * (aRR - aRL)) / (SAT - SAB);
-  E += T(SB_neg * ST_pos * SL_neg * SR_neg) * tmpE;
+  tmpE = quot_any(quot_any(SAL * SAB * EstarRR - SAL * SAT * EstarRL - SAR * SAB * EstarLR + SAR * SAT * EstarLL, iw),
+                  ih) -
+         quot(SAT * SAB, ih) * (AstarT - AstarB) + quot(SAR * SAL, iw) * (BstarR - BstarL);
+  E += on(!Bp && Tp && !Lp && Rp) * tmpE;
+  tmpE = quot_any(SAR * EstarLLx - SAL * EstarRLx + SAR * SAL * (bRL - bLL), iw);
+  tmpE = on(Lp) * ELL + on(!Lp && !Rp) * ERL + on(!Lp && Rp) * tmpE;
+  E += on(Bp) * tmpE;
+  tmpE = quot_any(SAR * EstarLRx - SAL * EstarRRx + SAR * SAL * (bRR - bLR), iw);
+  tmpE = on(Lp) * ELR + on(!Lp && !Rp) * ERR + on(!Lp && Rp) * tmpE;
+  E += on(!Bp && !Tp) * tmpE;
+  tmpE = quot_any(SAT * EstarLLy - SAB * EstarLRy - SAT * SAB * (aLR - aLL), ih);
+  E += on(!Bp && Tp && Lp) * tmpE;
+  tmpE = quot_any(SAT * EstarRLy - SAB * EstarRRy - SAT * SAB * (aRR - aRL), ih);
+  E += on(!Bp && Tp && !Lp && !Rp) * tmpE;
   return E;
 }
 
@@ -668,9 +690,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
     const T dBy = T(0.5) * (BR - BL);
     const T gamma = gas.gamma0;
     const T sr0 = (-u * drx - dux * r) * dtdx + (-v * dry - dvy * r) * dtdy;
-    const T su0 = (-u * dux - dpx / r - B * dBx / r - C * dCx / r) * dtdx + (-v * duy + B * dAy / r) * dtdy;
-    const T sv0 = (-u * dvx + A * dBx / r) * dtdx + (-v * dvy - dpy / r - A * dAy / r - C * dCy / r) * dtdy;
-    const T sw0 = (-u * dwx + A * dCx / r) * dtdx + (-v * dwy + B * dCy / r) * dtdy;
+    const Inv<T> ir = inv_of(r);
+    const T su0 = (-u * dux - quot(dpx, ir) - quot_any(B * dBx, ir) - quot_any(C * dCx, ir)) * dtdx +
+                  (-v * duy + quot_any(B * dAy, ir)) * dtdy;
+    const T sv0 = (-u * dvx + quot_any(A * dBx, ir)) * dtdx +
+                  (-v * dvy - quot(dpy, ir) - quot_any(A * dAy, ir) - quot_any(C * dCy, ir)) * dtdy;
+    const T sw0 = (-u * dwx + quot_any(A * dCx, ir)) * dtdx + (-v * dwy + quot_any(B * dCy, ir)) * dtdy;
     const T sp0 = (-u * dpx - dux * gamma * p) * dtdx + (-v * dpy - dvy * gamma * p) * dtdy;
     const T sA0 = (u * dBy + B * duy - v * dAy - A * dvy) * dtdy;
     const T sB0 = (-u * dBx - B * dux + v * dAx + A * dvx) * dtdx;

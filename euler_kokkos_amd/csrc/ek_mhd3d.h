@@ -272,12 +272,14 @@ __device__ __forceinline__ void trace_record(const TraceIn<T>& in, const Gas<T>&
   const T dAx = h * (AR - AL), dBy = h * (BR - BL), dCz = h * (CR - CL);
   const T gamma = gas.gamma0;
   const T sr0 = (-u * drx - dux * r) * dtdx + (-v * dry - dvy * r) * dtdy + (-ww * drz - dwz * r) * dtdz;
-  const T su0 = (-u * dux - (dpx + B * dBx + C * dCx) / r) * dtdx + (-v * duy + B * dAy / r) * dtdy +
-                (-ww * duz + C * dAz / r) * dtdz;
-  const T sv0 = (-u * dvx + A * dBx / r) * dtdx + (-v * dvy - (dpy + A * dAy + C * dCy) / r) * dtdy +
-                (-ww * dvz + C * dBz / r) * dtdz;
-  const T sw0 = (-u * dwx + A * dCx / r) * dtdx + (-v * dwy + B * dCy / r) * dtdy +
-                (-ww * dwz - (dpz + A * dAz + B * dBz) / r) * dtdz;
+  const Inv<T> ir = inv_of(r);
+  // (plain: in FP32 the y and z terms fuse into the sum, the x term's product is rounded)
+  const T su0 = plain((-u * dux - quot_any(dpx + B * dBx + C * dCx, ir)) * dtdx) +
+                (-v * duy + quot_any(B * dAy, ir)) * dtdy + (-ww * duz + quot_any(C * dAz, ir)) * dtdz;
+  const T sv0 = (-u * dvx + quot_any(A * dBx, ir)) * dtdx + (-v * dvy - quot_any(dpy + A * dAy + C * dCy, ir)) * dtdy +
+                (-ww * dvz + quot_any(C * dBz, ir)) * dtdz;
+  const T sw0 = (-u * dwx + quot_any(A * dCx, ir)) * dtdx + (-v * dwy + quot_any(B * dCy, ir)) * dtdy +
+                (-ww * dwz - quot_any(dpz + A * dAz + B * dBz, ir)) * dtdz;
   const T sp0 = (-u * dpx - dux * gamma * p) * dtdx + (-v * dpy - dvy * gamma * p) * dtdy +
                 (-ww * dpz - dwz * gamma * p) * dtdz;
   const T sA0 = (u * dBy + B * duy - v * dAy - A * dvy) * dtdy + (u * dCz + C * duz - ww * dAz - A * dwz) * dtdz;
@@ -579,16 +581,18 @@ __device__ __forceinline__ double cfl3(const Gas<T>& gas, const T* u, T mx, T my
     constoprim<T>(gas, u, mx, my, mz, q);
     const T d = q[ID], p = q[IP], a = q[IA], b = q[IB], c = q[IC];
     const T b2 = a * a + b * b + c * c;
-    const T c2 = gas.gamma0 * p / d;
-    const T d2 = T(0.5) * (b2 / d + c2);
-    const T vx = esqrt(d2 + esqrt(d2 * d2 - c2 * a * a / d)) + eabs(q[IU]);
-    const T vy = esqrt(d2 + esqrt(d2 * d2 - c2 * b * b / d)) + eabs(q[IV]);
-    const T vz = esqrt(d2 + esqrt(d2 * d2 - c2 * c * c / d)) + eabs(q[IW]);
+    const Inv<T> id = inv_of(d);
+    const T c2 = quot(gas.gamma0 * p, id);
+    const T d2 = T(0.5) * (quot(b2, id) + c2);
+    const T vx = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * a * a, id))) + eabs(q[IU]);
+    const T vy = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * b * b, id))) + eabs(q[IV]);
+    const T vz = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * c * c, id))) + eabs(q[IW]);
     if (geo.pow2)
       return vx * geo.idx + vy * geo.idy + vz * geo.idz;
-    return vx / geo.dx + vy / geo.dy + vz / geo.dz;
+    return quot(vx, inv_with(geo.dx, geo.rdx)) + quot(vy, inv_with(geo.dy, geo.rdy)) +
+           quot(vz, inv_with(geo.dz, geo.rdz));
   } else {
-    return mhd_cfl_widened<3>(gas, u, (double)mx, (double)my, (double)mz, geo.dx, geo.dy, geo.dz);
+    return mhd_cfl_widened<3>(gas, u, (double)mx, (double)my, (double)mz, geo.rdx, geo.rdy, geo.rdz);
   }
 }
 
