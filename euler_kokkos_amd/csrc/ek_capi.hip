@@ -357,17 +357,17 @@ static hipError_t launch_inv_dt_into(ek_ctx* c, unsigned long long* dst, unsigne
 {
   if (c->p.mhd && c->p.dim == 3) {
     if (c->p.precision == EK_FP64)
-      return ek::fp64::mhd3_inv_dt((const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, c->stream);
-    return ek::fp32::mhd3_inv_dt((const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, c->stream);
+      return ek::fp64::mhd3_inv_dt((const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, ek::NSPREAD, c->stream);
+    return ek::fp32::mhd3_inv_dt((const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, ek::NSPREAD, c->stream);
   }
   if (c->p.mhd) {
     if (c->p.precision == EK_FP64)
-      return ek::fp64::mhd_inv_dt((const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, c->stream);
-    return ek::fp32::mhd_inv_dt((const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, c->stream);
+      return ek::fp64::mhd_inv_dt((const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, ek::NSPREAD, c->stream);
+    return ek::fp32::mhd_inv_dt((const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, ek::NSPREAD, c->stream);
   }
   if (c->p.precision == EK_FP64)
-    return ek::fp64::inv_dt(c->p.dim, (const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, c->stream);
-  return ek::fp32::inv_dt(c->p.dim, (const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, c->stream);
+    return ek::fp64::inv_dt(c->p.dim, (const double*)c->U[c->cur], c->g64, c->gas64, dst, spread, ek::NSPREAD, c->stream);
+  return ek::fp32::inv_dt(c->p.dim, (const float*)c->U[c->cur], c->g32, c->gas32, dst, spread, ek::NSPREAD, c->stream);
 }
 
 extern "C" int ek_inv_dt(ek_ctx* c, double* inv_dt)
@@ -418,6 +418,7 @@ extern "C" int ek_step(ek_ctx* c, double dt)
   ek::StepCtl ctl{};
   ctl.ts = c->ts;
   ctl.spread = c->spread;
+  ctl.nspread = ek::NSPREAD;
   ctl.slot = 0;
   ctl.mode = 1;
   ctl.dt_given = dt;
@@ -444,6 +445,7 @@ static int build_graph(ek_ctx* c, int s, int nStepmax, double tEnd)
     ek::StepCtl ctl{};
     ctl.ts = c->ts;
     ctl.spread = c->spread;
+    ctl.nspread = ek::NSPREAD;
     ctl.slot = i % 3;
     ctl.mode = 0;
     ctl.cfl = c->p.cfl;
@@ -509,6 +511,7 @@ extern "C" int ek_run(ek_ctx* c, int nsteps, int nStepmax, double tEnd, double* 
     ek::StepCtl ctl{};
     ctl.ts = c->ts;
     ctl.spread = c->spread;
+    ctl.nspread = ek::NSPREAD;
     ctl.slot = r % 3;
     ctl.mode = 0;
     ctl.cfl = c->p.cfl;
@@ -739,6 +742,7 @@ extern "C" int ek_run_noalloc(const ek_params* params, void* U, void* U2, int ns
     ek::StepCtl ctl{};
     ctl.ts = c.ts;
     ctl.spread = c.spread;
+    ctl.nspread = ek::NSPREAD;
     ctl.slot = r % 3;
     ctl.mode = 0;
     ctl.cfl = c.p.cfl;

@@ -32,6 +32,7 @@ struct TimeSlot {
 struct StepCtl {
   TimeSlot* ts;
   unsigned long long* spread; // extra CFL words of the slots (see invdt_word), or null
+  int nspread;     // words per slot, a power of two up to 64 (unused without spread)
   int slot;        // slot this launch reads
   int mode;        // 0: dt = cfl/invdt (clamped to tEnd), 1: dt = dt_given
   double dt_given;
@@ -170,39 +171,42 @@ __device__ __forceinline__ double wave_max(double v)
 // CFL words of a time slot. Every block of a step ends with one device-scope atomic max,
 // and such atomics on one address serialize: with thousands of blocks per launch that cost
 // up to three quarters of a kernel's time. With StepCtl::spread set, the maximum of slot s
-// lives in NSPREAD words 256 bytes apart -- ts[s].invdt_bits (key 0) and
-// spread[(s*NSPREAD + k)*SPREAD_STRIDE] for k = 1..NSPREAD-1 -- block b updates word
-// b % NSPREAD and readers take the max of all of them. Max is exact, so dt is unchanged.
+// lives in n = StepCtl::nspread words 256 bytes apart -- ts[s].invdt_bits (key 0) and
+// spread[(s*n + k)*SPREAD_STRIDE] for k = 1..n-1 -- block b updates word b % n and readers
+// take the max of all of them. Max is exact, so dt is unchanged. The single-grid steps use
+// NSPREAD words.
 constexpr int NSPREAD = 64;
 constexpr int SPREAD_STRIDE = 32;
 constexpr long long SPREAD_ELEMS = 3LL * NSPREAD * SPREAD_STRIDE;
 
 __device__ __forceinline__ unsigned long long* invdt_word(const StepCtl& c, int slot, unsigned key)
 {
-  const unsigned k = key & (NSPREAD - 1);
+  const unsigned k = key & (unsigned)(c.nspread - 1);
   if (!c.spread || k == 0)
     return &c.ts[slot].invdt_bits;
-  return c.spread + ((long long)slot * NSPREAD + k) * SPREAD_STRIDE;
+  return c.spread + ((long long)slot * c.nspread + k) * SPREAD_STRIDE;
 }
 
 // Max over the words of `slot`; `own` is ts[slot].invdt_bits as already read. Call with
 // the whole wave active (lane k reads word k).
 __device__ __forceinline__ unsigned long long invdt_gather(const StepCtl& c, int slot, unsigned long long own)
 {
-  static_assert(NSPREAD == 64, "one word per lane");
+  static_assert(NSPREAD <= 64, "one word per lane");
   if (!c.spread)
     return own;
   const int lane = threadIdx.x & 63;
-  const unsigned long long v =
-      lane == 0 ? own : c.spread[((long long)slot * NSPREAD + lane) * SPREAD_STRIDE];
+  unsigned long long v = own;
+  if (lane > 0 && lane < c.nspread)
+    v = c.spread[((long long)slot * c.nspread + lane) * SPREAD_STRIDE];
   return wave_umax(v);
 }
 
-// Word of block blockIdx.x in a standalone CFL reduction: dst itself, or, with spread
-// words (spread + k*SPREAD_STRIDE for k = 1..NSPREAD-1, k = 0 being dst), word b % NSPREAD.
-__device__ __forceinline__ unsigned long long* reduce_word(unsigned long long* dst, unsigned long long* spread)
+// Word of block blockIdx.x in a standalone CFL reduction: dst itself, or, with nspread spread
+// words (spread + k*SPREAD_STRIDE for k = 1..nspread-1, k = 0 being dst), word b % nspread.
+__device__ __forceinline__ unsigned long long* reduce_word(unsigned long long* dst, unsigned long long* spread,
+                                                           int nspread)
 {
-  const unsigned k = blockIdx.x & (NSPREAD - 1);
+  const unsigned k = blockIdx.x & (unsigned)(nspread - 1);
   return (spread && k) ? spread + (long long)k * SPREAD_STRIDE : dst;
 }
 
@@ -271,8 +275,8 @@ __device__ __forceinline__ void step_end_bookkeeping(const StepCtl& c, const Tim
     c.ts[nxt].it = cur.it + 1;
     c.ts[nxt].finished = 0;
     c.ts[nn].invdt_bits = 0ull;
-  } else if (c.spread) {
-    c.spread[((long long)nn * NSPREAD + lane) * SPREAD_STRIDE] = 0ull;
+  } else if (c.spread && lane < c.nspread) {
+    c.spread[((long long)nn * c.nspread + lane) * SPREAD_STRIDE] = 0ull;
   }
 }
 
@@ -494,7 +498,7 @@ __global__ __launch_bounds__(NT) void hydro2d_step(const T* __restrict__ Uin, T*
 template <class T, int DIM, int NT>
 __global__ __launch_bounds__(NT) void inv_dt_kernel(const T* __restrict__ U, Geom<T> geo, Gas<T> gas,
                                                     unsigned long long* dst, unsigned long long* spread,
-                                                    long long ncell)
+                                                    int nspread, long long ncell)
 {
   __shared__ double sred[NT / 64];
   constexpr int NV = DIM == 3 ? 5 : 4;
@@ -507,7 +511,7 @@ __global__ __launch_bounds__(NT) void inv_dt_kernel(const T* __restrict__ U, Geo
     const double s = cfl_term<T, DIM>(gas, u, geo);
     local = (s > local || !(s == s)) ? s : local;
   }
-  block_max_to<NT>(reduce_word(dst, spread), local, sred);
+  block_max_to<NT>(reduce_word(dst, spread, nspread), local, sred);
 }
 
 // Compensated (Neumaier) FP64 sums of each conserved variable over the interior:

@@ -1095,7 +1095,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
 // the boundary map when they are ghosts.
 template <class T, int NT>
 __global__ __launch_bounds__(NT) void mhd2d_inv_dt_kernel(const T* __restrict__ U, Geom<T> geo, Gas<T> gas,
-                                                           unsigned long long* dst, unsigned long long* spread)
+                                                           unsigned long long* dst, unsigned long long* spread,
+                                                      int nspread)
 {
   __shared__ double sred[NT / 64];
   const long long ncell = geo.vstride;
@@ -1120,7 +1121,7 @@ __global__ __launch_bounds__(NT) void mhd2d_inv_dt_kernel(const T* __restrict__ 
     const double s = mhd_cfl_term<T>(gas, u, mx, my, geo);
     local = (s > local || !(s == s)) ? s : local;
   }
-  block_max_to<NT>(reduce_word(dst, spread), local, sred);
+  block_max_to<NT>(reduce_word(dst, spread, nspread), local, sred);
 }
 
 } // namespace mhd

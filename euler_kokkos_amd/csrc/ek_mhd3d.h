@@ -705,7 +705,8 @@ __global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ S, T*
 // boundary map
 template <class T>
 __global__ __launch_bounds__(256) void inv_dt3_kernel(const T* __restrict__ U, Geom<T> geo, Gas<T> gas,
-                                                      unsigned long long* dst, unsigned long long* spread)
+                                                      unsigned long long* dst, unsigned long long* spread,
+                                                      int nspread)
 {
   __shared__ double sred[4];
   const long long n = geo.vstride;
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(256) void inv_dt3_kernel(const T* __restrict__ U, G
     const double s = cfl3<T>(gas, u, mx, my, mz, geo);
     local = (s > local || !(s == s)) ? s : local;
   }
-  block_max_to<256>(reduce_word(dst, spread), local, sred);
+  block_max_to<256>(reduce_word(dst, spread, nspread), local, sred);
 }
 
 } // namespace mhd3

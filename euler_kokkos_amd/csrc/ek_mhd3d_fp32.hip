@@ -45,12 +45,13 @@ hipError_t mhd3_step(int rs, int st, const float* Uin, float* Uout, float* scrat
 }
 
 hipError_t mhd3_inv_dt(const float* U, const Geom<float>& geo, const Gas<float>& gas, unsigned long long* dst,
-                       unsigned long long* spread, hipStream_t s)
+                       unsigned long long* spread, int nspread,
+                  hipStream_t s)
 {
   long long nb = (geo.vstride + 255) / 256;
   if (nb > 4096)
     nb = 4096;
-  hipLaunchKernelGGL(mhd3::inv_dt3_kernel<float>, dim3((unsigned)nb), dim3(256), 0, s, U, geo, gas, dst, spread);
+  hipLaunchKernelGGL(mhd3::inv_dt3_kernel<float>, dim3((unsigned)nb), dim3(256), 0, s, U, geo, gas, dst, spread, nspread);
   return hipGetLastError();
 }
 

@@ -45,12 +45,13 @@ hipError_t mhd3_step(int rs, int st, const double* Uin, double* Uout, double* sc
 }
 
 hipError_t mhd3_inv_dt(const double* U, const Geom<double>& geo, const Gas<double>& gas, unsigned long long* dst,
-                       unsigned long long* spread, hipStream_t s)
+                       unsigned long long* spread, int nspread,
+                  hipStream_t s)
 {
   long long nb = (geo.vstride + 255) / 256;
   if (nb > 4096)
     nb = 4096;
-  hipLaunchKernelGGL(mhd3::inv_dt3_kernel<double>, dim3((unsigned)nb), dim3(256), 0, s, U, geo, gas, dst, spread);
+  hipLaunchKernelGGL(mhd3::inv_dt3_kernel<double>, dim3((unsigned)nb), dim3(256), 0, s, U, geo, gas, dst, spread, nspread);
   return hipGetLastError();
 }
 

@@ -37,6 +37,9 @@ struct HostJob {
 
 constexpr long long kAlign = 64; // elements
 constexpr int kGraphSteps = 6;   // lcm of the 2 arena buffers and the 3 time slots
+// job slots with their own spread CFL words (12 KiB each); a pool with more jobs than this has
+// so many tiles of other jobs in flight that one word per job is enough for the rest
+constexpr int kSpreadJobs = 2048;
 constexpr int kCz[4] = { 8, 16, 32, 64 };
 // 3D MHD pools: share of the arena for the two state buffers; the rest is the work buffer
 // (78 reals per ghost-padded cell against 2 x 8 per cell: 13-16 % for edges 64-192)
@@ -68,7 +71,7 @@ struct ek_pool {
   long long nstep = 0;
   int variant = 0;
   int cus = 1;
-  int grid = 1;
+  unsigned long long* spread = nullptr; // hydro: POOL_SPREAD_ELEMS CFL words of each of the first kSpreadJobs job slots
   hipGraphExec_t graph = nullptr;
   bool graph_ok = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -132,6 +135,18 @@ static int cz_of(const ek_pool* p, const ek_params& j)
   return (j.nz + nch - 1) / nch;
 }
 
+// Spread CFL words of job `id` (StepCtl::spread), or null
+static unsigned long long* spread_of(const ek_pool* p, int id)
+{
+  return p->spread && id < kSpreadJobs ? p->spread + (size_t)id * ek::POOL_SPREAD_ELEMS : nullptr;
+}
+
+// bytes of all of them
+static size_t spread_bytes(const ek_pool* p)
+{
+  return p->mhd3 ? 0 : (size_t)std::min(p->max_jobs, kSpreadJobs) * ek::POOL_SPREAD_ELEMS * sizeof(unsigned long long);
+}
+
 // PoolJob record of job `id` for the current tile choice
 template <class T>
 static ek::PoolJob<T> make_record(const ek_pool* p, int id)
@@ -142,6 +157,7 @@ static ek::PoolJob<T> make_record(const ek_pool* p, int id)
   r.slot0 = 3 * id;
   r.nStepmax = h.nStepmax;
   r.cz = h.p.dim == 3 ? cz_of(p, h.p) : 1;
+  r.spread = spread_of(p, id);
   r.cfl = h.p.cfl;
   r.tEnd = h.tEnd;
   ek::fill_geom<T>(h.p, r.geo, r.gas);
@@ -304,12 +320,7 @@ static void set_grid(ek_pool* p)
       ek::fp64::pool_mhd3_grids(rs, st, p->cus, p->mgrid);
     else
       ek::fp32::pool_mhd3_grids(rs, st, p->cus, p->mgrid);
-    p->grid = p->mgrid[0];
-    return;
   }
-  const int occ = p->fp64 ? ek::fp64::pool_occupancy(kind_dim(p), p->variant, (int)p->kind.slope_type)
-                          : ek::fp32::pool_occupancy(kind_dim(p), p->variant, (int)p->kind.slope_type);
-  p->grid = p->cus * occ;
 }
 
 static hipError_t launch_one(ek_pool* p, long long n)
@@ -328,11 +339,9 @@ static hipError_t launch_one(ek_pool* p, long long n)
   }
   if (p->fp64)
     return ek::fp64::pool_step(kind_dim(p), p->variant, st, (const double*)p->A[par], (double*)p->A[1 - par],
-                               (const ek::PoolJob<double>*)p->djobs, p->dwork, p->nwork, p->ts, slot, p->grid,
-                               p->stream);
+                               (const ek::PoolJob<double>*)p->djobs, p->dwork, p->nwork, p->ts, slot, p->stream);
   return ek::fp32::pool_step(kind_dim(p), p->variant, st, (const float*)p->A[par], (float*)p->A[1 - par],
-                             (const ek::PoolJob<float>*)p->djobs, p->dwork, p->nwork, p->ts, slot, p->grid,
-                             p->stream);
+                             (const ek::PoolJob<float>*)p->djobs, p->dwork, p->nwork, p->ts, slot, p->stream);
 }
 
 static int capture_graph(ek_pool* p)
@@ -500,6 +509,7 @@ extern "C" int ek_pool_create(const ek_params* kind, long long arena_bytes, int 
       (mhd3 && (e = hipMalloc(&p->W, (size_t)p->wcap * p->elem)) != hipSuccess) ||
       (e = hipMalloc(&p->ts, (size_t)max_jobs * 3 * sizeof(ek::TimeSlot))) != hipSuccess ||
       (e = hipMalloc(&p->djobs, (size_t)max_jobs * recb)) != hipSuccess ||
+      (spread_bytes(p) && (e = hipMalloc(&p->spread, spread_bytes(p))) != hipSuccess) ||
       (e = hipMalloc(&p->partial, (size_t)1024 * 16 * sizeof(double))) != hipSuccess ||
       (e = hipEventCreate(&p->ev0)) != hipSuccess || (e = hipEventCreate(&p->ev1)) != hipSuccess ||
       (e = hipMemsetAsync(p->ts, 0, (size_t)max_jobs * 3 * sizeof(ek::TimeSlot), p->stream)) != hipSuccess ||
@@ -534,6 +544,7 @@ extern "C" void ek_pool_destroy(ek_pool* p)
   hipFree(p->A[1]);
   hipFree(p->ts);
   hipFree(p->djobs);
+  hipFree(p->spread);
   hipFree(p->dwork);
   hipFree(p->dworkU);
   hipFree(p->W);
@@ -645,23 +656,29 @@ static int admit_upload(ek_pool* p, const ek_params* jp, const double* host, int
 static int init_slots(ek_pool* p, const ek_params* jp, int id, const char* dst)
 {
   PHIP(p, hipMemcpyAsync(p->ts + 3 * id, p->zslots, sizeof(p->zslots), hipMemcpyHostToDevice, p->stream));
-  unsigned long long* bits = &p->ts[3 * id + (int)(p->nstep % 3)].invdt_bits;
+  const int slot = (int)(p->nstep % 3);
+  unsigned long long* bits = &p->ts[3 * id + slot].invdt_bits;
+  unsigned long long* spread = spread_of(p, id);
+  if (spread) {
+    PHIP(p, hipMemsetAsync(spread, 0, ek::POOL_SPREAD_ELEMS * sizeof(unsigned long long), p->stream));
+    spread += (size_t)slot * ek::POOL_NSPREAD * ek::SPREAD_STRIDE;
+  }
   if (p->fp64) {
     ek::Geom<double> g;
     ek::Gas<double> gs;
     ek::fill_geom<double>(*jp, g, gs);
     if (p->mhd3)
-      PHIP(p, ek::fp64::mhd3_inv_dt((const double*)dst, g, gs, bits, nullptr, p->stream));
+      PHIP(p, ek::fp64::mhd3_inv_dt((const double*)dst, g, gs, bits, nullptr, 1, p->stream));
     else
-      PHIP(p, ek::fp64::inv_dt(jp->dim, (const double*)dst, g, gs, bits, nullptr, p->stream));
+      PHIP(p, ek::fp64::inv_dt(jp->dim, (const double*)dst, g, gs, bits, spread, ek::POOL_NSPREAD, p->stream));
   } else {
     ek::Geom<float> g;
     ek::Gas<float> gs;
     ek::fill_geom<float>(*jp, g, gs);
     if (p->mhd3)
-      PHIP(p, ek::fp32::mhd3_inv_dt((const float*)dst, g, gs, bits, nullptr, p->stream));
+      PHIP(p, ek::fp32::mhd3_inv_dt((const float*)dst, g, gs, bits, nullptr, 1, p->stream));
     else
-      PHIP(p, ek::fp32::inv_dt(jp->dim, (const float*)dst, g, gs, bits, nullptr, p->stream));
+      PHIP(p, ek::fp32::inv_dt(jp->dim, (const float*)dst, g, gs, bits, spread, ek::POOL_NSPREAD, p->stream));
   }
   return EK_OK;
 }
@@ -1047,16 +1064,20 @@ extern "C" int ek_pool_autotune(ek_pool* p, int steps, int* choice, double* ms_o
   if (int rc = activate_pending(p, 2)) // the snapshot below holds every job's state
     return rc;
   const int nvar = p->mhd3 ? 1 : (p->kind.dim == 2 ? ek::pool::N2VARIANTS : 4);
-  // snapshot of the current buffer and the time slots, restored after every trial
+  // snapshot of the current buffer, the time slots and the CFL words, restored after every trial
   long long hi = 0;
   for (const HostJob& h : p->jobs)
     if (h.used)
       hi = std::max(hi, h.off + h.alloc);
   void* snap = nullptr;
   ek::TimeSlot* tsnap = nullptr;
+  void* wsnap = nullptr;
   const size_t sbytes = (size_t)hi * p->elem, tbytes = (size_t)p->max_jobs * 3 * sizeof(ek::TimeSlot);
-  if (hipMalloc(&snap, sbytes ? sbytes : 8) != hipSuccess || hipMalloc(&tsnap, tbytes) != hipSuccess) {
+  const size_t wbytes = spread_bytes(p);
+  if (hipMalloc(&snap, sbytes ? sbytes : 8) != hipSuccess || hipMalloc(&tsnap, tbytes) != hipSuccess ||
+      (wbytes && hipMalloc(&wsnap, wbytes) != hipSuccess)) {
     hipFree(snap);
+    hipFree(tsnap);
     return pfail(p, EK_ENOMEM, "autotune snapshot allocation failed");
   }
   const int par = (int)(p->nstep % 2);
@@ -1067,6 +1088,8 @@ extern "C" int ek_pool_autotune(ek_pool* p, int steps, int* choice, double* ms_o
     hipError_t e = hipMemcpyAsync(p->A[par], snap, sbytes, hipMemcpyDeviceToDevice, p->stream);
     if (e == hipSuccess)
       e = hipMemcpyAsync(p->ts, tsnap, tbytes, hipMemcpyDeviceToDevice, p->stream);
+    if (e == hipSuccess && wbytes)
+      e = hipMemcpyAsync(p->spread, wsnap, wbytes, hipMemcpyDeviceToDevice, p->stream);
     if (e == hipSuccess)
       e = hipStreamSynchronize(p->stream);
     return e;
@@ -1074,6 +1097,8 @@ extern "C" int ek_pool_autotune(ek_pool* p, int steps, int* choice, double* ms_o
   hipError_t e = hipMemcpyAsync(snap, p->A[par], sbytes, hipMemcpyDeviceToDevice, p->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(tsnap, p->ts, tbytes, hipMemcpyDeviceToDevice, p->stream);
+  if (e == hipSuccess && wbytes)
+    e = hipMemcpyAsync(wsnap, p->spread, wbytes, hipMemcpyDeviceToDevice, p->stream);
   if (e == hipSuccess)
     e = hipStreamSynchronize(p->stream);
   for (int v = 0; v < nvar && e == hipSuccess && rc == EK_OK; v++) {
@@ -1104,6 +1129,7 @@ extern "C" int ek_pool_autotune(ek_pool* p, int steps, int* choice, double* ms_o
   }
   hipFree(snap);
   hipFree(tsnap);
+  hipFree(wsnap);
   if (e != hipSuccess)
     return pfail(p, EK_EHIP, std::string("autotune: ") + hipGetErrorString(e));
   if (rc)

@@ -5,13 +5,9 @@
 namespace ek {
 namespace fp64 {
 hipError_t pool_step(int dim, int variant, int st, const double* Ua, double* Ub, const PoolJob<double>* jobs,
-                     const PoolWork* work, int nwork, TimeSlot* ts, int slot, int grid, hipStream_t s)
+                     const PoolWork* work, int nwork, TimeSlot* ts, int slot, hipStream_t s)
 {
-  return pool::launch_step<double>(dim, variant, st, Ua, Ub, jobs, work, nwork, ts, slot, grid, s);
-}
-int pool_occupancy(int dim, int variant, int st)
-{
-  return pool::occupancy<double>(dim, variant, st);
+  return pool::launch_step<double>(dim, variant, st, Ua, Ub, jobs, work, nwork, ts, slot, s);
 }
 } // namespace fp64
 } // namespace ek

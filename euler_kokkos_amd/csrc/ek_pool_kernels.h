@@ -1,12 +1,21 @@
-// ek_pool_kernels.h -- batched steps of many independent grids (a job pool) in one persistent launch.
+// ek_pool_kernels.h -- batched steps of many independent grids (a job pool) in one launch.
 //
 // Every job keeps its own state in a shared device arena (two ping-pong buffers, the job at
 // the same element offset in both), its own geometry, gas constants and time slots. One
-// launch advances every active job by one step of its own dt: the blocks walk a work list
-// of (job, tile) items and run the same per-tile code as the single-grid kernels
+// launch advances every active job by one step of its own dt: block b runs item b of a work
+// list of (job, tile) items with the same per-tile code as the single-grid kernels
 // (hydro2d_tile / hydro3d_column), so a job's results are those of its single-grid run.
 // Each job's first tile keeps that job's time bookkeeping; every tile reduces its CFL term
-// into the job's next slot.
+// into one of the job's CFL words (PoolJob::spread).
+//
+// A tile is short and starts with a chain of dependent reads (item, job record, time slot, CFL
+// words, cells), so what counts is how many tiles are in flight and how long their closing
+// atomics queue. One word per job made the atomics of a job's tiles serialize (about 70 ns
+// each): 24 blasts of edges 64-320 took 57 us per step, 256 of edges 64-512 682 us (FP32), 100
+// of them 564 us (FP64) in a persistent grid walking ranges of the list. With 16 words per job
+// (4 to 64 measured alike but for 64's longer reads), one block per item and the items in
+// XCD order (pool_item): 30, 617 and 496 us. 3D jobs (six of edges 64-160): 452 -> 324 us
+// FP32, 898 -> 709 us FP64.
 #pragma once
 
 #include "ek_hydro.h"
@@ -14,12 +23,17 @@
 
 namespace ek {
 
+// CFL words per slot of a job
+constexpr int POOL_NSPREAD = 16;
+constexpr long long POOL_SPREAD_ELEMS = 3LL * POOL_NSPREAD * SPREAD_STRIDE;
+
 template <class T>
 struct PoolJob {
   long long off;   // element offset of the job's state in each arena buffer
   int slot0;       // index of the job's first TimeSlot (3 per job)
   int nStepmax;
   int cz;          // z planes per column chunk (3D)
+  unsigned long long* spread; // the job's extra CFL words (POOL_SPREAD_ELEMS), or null
   int ntx, nty;    // tiles per axis
   double cfl, tEnd;
   Geom<T> geo;
@@ -32,49 +46,44 @@ struct PoolWork {
   int tz_first; // z chunk * 2 + (1 if this item does the job's bookkeeping)
 };
 
-// Items of block b: a contiguous range of the work list, so neighbouring tiles of a job run
-// one after the other on the same XCD (their halo lines meet in that XCD's L2).
-__device__ __forceinline__ void pool_range(int nwork, int& w0, int& w1)
+// Work item of this block: blocks are dealt to the 8 XCDs round robin, so each XCD gets a
+// contiguous eighth of the list and neighbouring tiles of a job share its L2 (33 -> 30 us for
+// the 24 blasts above; the remainder of the list keeps its order).
+__device__ __forceinline__ unsigned pool_item()
 {
-  const int per = nwork / (int)gridDim.x, rem = nwork % (int)gridDim.x;
-  const int b = blockIdx.x;
-  w0 = b * per + (b < rem ? b : rem);
-  w1 = w0 + per + (b < rem ? 1 : 0);
+  const unsigned n8 = gridDim.x / 8, b = blockIdx.x;
+  return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;
 }
 
 template <class T, int TX, int TY, int NT, int RS, int ST>
 __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
-                                                        const PoolWork* __restrict__ work, int nwork,
+                                                        const PoolWork* __restrict__ work,
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  int w0, w1;
-  pool_range(nwork, w0, w1);
-  for (int w = w0; w < w1; w++) {
-    const PoolWork it = work[w];
-    const PoolJob<T> J = jobs[it.job];
-    StepCtl ctl;
-    ctl.ts = ts + J.slot0;
-    ctl.spread = nullptr; // jobs' atomics already land on different slots
-    ctl.slot = slot;
-    ctl.mode = 0;
-    ctl.dt_given = 0.0;
-    ctl.cfl = J.cfl;
-    ctl.tEnd = J.tEnd;
-    ctl.nStepmax = J.nStepmax;
-    const bool first = (it.tz_first & 1) != 0;
-    double dt;
-    TimeSlot cur;
-    if (!step_begin(ctl, first, dt, cur))
-      continue;
-    __syncthreads(); // the previous item's shared-memory reads are done
-    const double local =
-        hydro2d_tile<T, TX, TY, NT, RS, ST>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt, it.tx * TX, it.ty * TY);
-    block_max_to<NT>(&ctl.ts[(slot + 1) % 3].invdt_bits, local, sred);
-    if (first && threadIdx.x < 64)
-      step_end_bookkeeping(ctl, cur, dt);
-  }
+  const PoolWork it = work[pool_item()];
+  const PoolJob<T> J = jobs[it.job];
+  StepCtl ctl;
+  ctl.ts = ts + J.slot0;
+  ctl.spread = J.spread;
+  ctl.nspread = POOL_NSPREAD;
+  ctl.slot = slot;
+  ctl.mode = 0;
+  ctl.dt_given = 0.0;
+  ctl.cfl = J.cfl;
+  ctl.tEnd = J.tEnd;
+  ctl.nStepmax = J.nStepmax;
+  const bool first = (it.tz_first & 1) != 0;
+  double dt;
+  TimeSlot cur;
+  if (!step_begin(ctl, first, dt, cur))
+    return;
+  const double local =
+      hydro2d_tile<T, TX, TY, NT, RS, ST>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt, it.tx * TX, it.ty * TY);
+  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
+  if (first && threadIdx.x < 64)
+    step_end_bookkeeping(ctl, cur, dt);
 }
 
 // Occupancy targets: FP64 3 waves per SIMD (what the shared memory allows anyway); FP32 5,
@@ -83,37 +92,33 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
 template <class T, int TX, int TY, int NT, int RS, int ST>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 5))) void hydro3d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
-                                                        const PoolWork* __restrict__ work, int nwork,
+                                                        const PoolWork* __restrict__ work,
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  int w0, w1;
-  pool_range(nwork, w0, w1);
-  for (int w = w0; w < w1; w++) {
-    const PoolWork it = work[w];
-    const PoolJob<T> J = jobs[it.job];
-    StepCtl ctl;
-    ctl.ts = ts + J.slot0;
-    ctl.spread = nullptr; // jobs' atomics already land on different slots
-    ctl.slot = slot;
-    ctl.mode = 0;
-    ctl.dt_given = 0.0;
-    ctl.cfl = J.cfl;
-    ctl.tEnd = J.tEnd;
-    ctl.nStepmax = J.nStepmax;
-    const bool first = (it.tz_first & 1) != 0;
-    double dt;
-    TimeSlot cur;
-    if (!step_begin(ctl, first, dt, cur))
-      continue;
-    __syncthreads();
-    const double local = hydro3d_column<T, TX, TY, NT, RS, ST, false>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt,
-                                                               it.tx * TX, it.ty * TY, (it.tz_first >> 1) * J.cz,
-                                                               J.cz);
-    block_max_to<NT>(&ctl.ts[(slot + 1) % 3].invdt_bits, local, sred);
-    if (first && threadIdx.x < 64)
-      step_end_bookkeeping(ctl, cur, dt);
-  }
+  const PoolWork it = work[pool_item()];
+  const PoolJob<T> J = jobs[it.job];
+  StepCtl ctl;
+  ctl.ts = ts + J.slot0;
+  ctl.spread = J.spread;
+  ctl.nspread = POOL_NSPREAD;
+  ctl.slot = slot;
+  ctl.mode = 0;
+  ctl.dt_given = 0.0;
+  ctl.cfl = J.cfl;
+  ctl.tEnd = J.tEnd;
+  ctl.nStepmax = J.nStepmax;
+  const bool first = (it.tz_first & 1) != 0;
+  double dt;
+  TimeSlot cur;
+  if (!step_begin(ctl, first, dt, cur))
+    return;
+  const double local = hydro3d_column<T, TX, TY, NT, RS, ST, false>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt,
+                                                             it.tx * TX, it.ty * TY, (it.tz_first >> 1) * J.cz,
+                                                             J.cz);
+  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
+  if (first && threadIdx.x < 64)
+    step_end_bookkeeping(ctl, cur, dt);
 }
 
 } // namespace ek

@@ -14,7 +14,7 @@ constexpr int V2[N2VARIANTS][3] = { { 16, 16, 256 }, { 32, 8, 256 }, { 16, 8, 12
 constexpr int P3X = 16, P3Y = 8, P3T = 256;
 
 template <class T>
-using Pool2Fn = void (*)(const T*, T*, const PoolJob<T>*, const PoolWork*, int, TimeSlot*, int);
+using Pool2Fn = void (*)(const T*, T*, const PoolJob<T>*, const PoolWork*, TimeSlot*, int);
 
 template <class T, int V, int ST>
 inline Pool2Fn<T> pick2v()
@@ -45,36 +45,17 @@ inline Pool2Fn<T> pick3(int st)
   return hydro3d_pool_step<T, P3X, P3Y, P3T, RS_HLLC, 2>;
 }
 
-// blocks of `variant` that fit on one CU at once
-template <class T>
-inline int occupancy(int dim, int variant, int st)
-{
-  int n = 0;
-  if (dim == 2) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(pick2<T>(variant, st)),
-                                                     V2[variant][2], 0) != hipSuccess)
-      return 1;
-  } else {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(pick3<T>(st)), P3T, 0) !=
-        hipSuccess)
-      return 1;
-  }
-  return n > 0 ? n : 1;
-}
-
 template <class T>
 inline hipError_t launch_step(int dim, int variant, int st, const T* Ua, T* Ub, const PoolJob<T>* jobs,
-                              const PoolWork* work, int nwork, TimeSlot* ts, int slot, int grid, hipStream_t s)
+                              const PoolWork* work, int nwork, TimeSlot* ts, int slot, hipStream_t s)
 {
   if (nwork <= 0)
     return hipSuccess;
-  if (grid > nwork)
-    grid = nwork;
   if (dim == 2)
-    hipLaunchKernelGGL(pick2<T>(variant, st), dim3(grid), dim3(V2[variant][2]), 0, s, Ua, Ub, jobs, work, nwork,
-                       ts, slot);
+    hipLaunchKernelGGL(pick2<T>(variant, st), dim3(nwork), dim3(V2[variant][2]), 0, s, Ua, Ub, jobs, work, ts,
+                       slot);
   else
-    hipLaunchKernelGGL(pick3<T>(st), dim3(grid), dim3(P3T), 0, s, Ua, Ub, jobs, work, nwork, ts, slot);
+    hipLaunchKernelGGL(pick3<T>(st), dim3(nwork), dim3(P3T), 0, s, Ua, Ub, jobs, work, ts, slot);
   return hipGetLastError();
 }
 

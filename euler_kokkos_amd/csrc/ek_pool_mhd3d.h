@@ -44,6 +44,7 @@ __device__ __forceinline__ StepCtl pool_ctl(const PoolJobM<T>& J, TimeSlot* ts, 
   StepCtl ctl;
   ctl.ts = ts + J.slot0;
   ctl.spread = nullptr;
+  ctl.nspread = 1;
   ctl.slot = slot;
   ctl.mode = 0;
   ctl.dt_given = 0.0;
@@ -122,6 +123,16 @@ __global__ __launch_bounds__(256) void mhd3_pool_fluxemf(T* __restrict__ W, cons
   pool_padded_unit<T, 4>(jobs, work, ts, slot, [&](const PoolJobM<T>& J, double, unsigned c, int task) {
     mhd3::fluxemf_cell<T, RS>(W + J.woff, J.w, J.gas, c, task);
   });
+}
+
+// Items of block b: a contiguous range of the work list, so neighbouring tiles of a job run
+// one after the other on the same XCD (their halo lines meet in that XCD's L2).
+__device__ __forceinline__ void pool_range(int nwork, int& w0, int& w1)
+{
+  const int per = nwork / (int)gridDim.x, rem = nwork % (int)gridDim.x;
+  const int b = blockIdx.x;
+  w0 = b * per + (b < rem ? b : rem);
+  w1 = w0 + per + (b < rem ? 1 : 0);
 }
 
 // Update. A block's range holds consecutive units of few jobs: the block keeps a running CFL

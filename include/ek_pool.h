@@ -10,12 +10,12 @@
  *
  * Jobs live in a fixed device arena (two ping-pong buffers); admission reserves the job's
  * state in both, retirement frees it. One ek_pool_step launch advances every unfinished
- * job by one step of its own dt, walking a work list of (job, tile) items with a
- * persistent grid; consecutive steps over an unchanged job set are replayed from a
+ * job by one step of its own dt, one block per (job, tile) item of a work
+ * list; consecutive steps over an unchanged job set are replayed from a
  * captured HIP graph. Tile shapes are chosen by ek_pool_autotune. A 3D MHD pool also keeps
  * each job's ghost-padded work area (78 reals per padded cell) in a work buffer that takes
  * 84 % of arena_bytes (the two state buffers take the rest), and one pool step is the five
- * kernels of the 3D MHD step, each a persistent grid over all active jobs.
+ * kernels of the 3D MHD step, each over all active jobs.
  *
  * All calls return 0 or an EK_E* code (include/ek_hip.h) with a message from
  * ek_pool_last_error. One pool per host thread.
