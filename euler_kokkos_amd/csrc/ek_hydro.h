@@ -210,6 +210,17 @@ __device__ __forceinline__ unsigned long long* reduce_word(unsigned long long* d
   return (spread && k) ? spread + (long long)k * SPREAD_STRIDE : dst;
 }
 
+// Position of block b of n in an order that gives each XCD a contiguous eighth of the grid
+// (blocks are dealt to the 8 XCDs round robin; the remainder keeps its place): neighbouring
+// tiles then share their halo lines in one XCD's L2 (per step, same box, in dispatch order ->
+// in this one: 2D hydro 64^2 9.6 -> 9.4 us, 512^2 19.8 -> 18.2, 1000x333 FP32 two-shock 18.5
+// -> 14.6; 2D MHD 300x211 26.0 -> 22.8, 1024^2 210 -> 206, FP32 84.1 -> 81.9).
+__device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
+{
+  const unsigned n8 = n / 8;
+  return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;
+}
+
 // Block max then one atomic per block. NaN (a failed cell) wins: its bit pattern is above
 // every finite double's, so a blown-up state yields dt = NaN instead of being skipped.
 template <int NT>
@@ -480,14 +491,16 @@ __global__ __launch_bounds__(NT) void hydro2d_step(const T* __restrict__ Uin, T*
                                                    Geom<T> geo, Gas<T> gas, StepCtl ctl)
 {
   __shared__ double sred[NT / 64];
-  const bool first_block = blockIdx.x == 0 && blockIdx.y == 0;
+  const bool first_block = blockIdx.x == 0;
+  const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(geo.nx + TX - 1) / TX;
+  const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
   double dt;
   TimeSlot cur;
   if (!step_begin(ctl, first_block, dt, cur))
     return;
   const double local =
-      hydro2d_tile<T, TX, TY, NT, RS, ST>(Uin, Uout, geo, gas, dt, blockIdx.x * TX, blockIdx.y * TY);
-  block_max_to<NT>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x + blockIdx.y * gridDim.x), local, sred);
+      hydro2d_tile<T, TX, TY, NT, RS, ST>(Uin, Uout, geo, gas, dt, i0, j0);
+  block_max_to<NT>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x), local, sred);
   if (first_block && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);
 }

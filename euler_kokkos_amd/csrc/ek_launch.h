@@ -49,7 +49,7 @@ inline hipError_t launch_step(int dim, int rs, int st, const T* Uin, T* Uout, co
       case RS_HLL: f = pick2<T, RS_HLL>(st); break;
       default: f = pick2<T, RS_HLLC>(st); break;
     }
-    dim3 grid((geo.nx + T2X - 1) / T2X, (geo.ny + T2Y - 1) / T2Y, 1);
+    dim3 grid((unsigned)((geo.nx + T2X - 1) / T2X) * (unsigned)((geo.ny + T2Y - 1) / T2Y));
     hipLaunchKernelGGL(f, grid, dim3(N2T), 0, s, Uin, Uout, geo, gas, ctl);
   } else {
     Step3Fn<T> f;

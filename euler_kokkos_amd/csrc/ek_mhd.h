@@ -564,7 +564,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
   T* const sDBx = sBev + L::BYN;         // [BYN] transverse slope dB/dx at y faces (halved)
 
   const int tid = threadIdx.x;
-  const bool first_block = blockIdx.x == 0 && blockIdx.y == 0;
+  const bool first_block = blockIdx.x == 0;
   double dt;
   TimeSlot cur;
   if (!step_begin(ctl, first_block, dt, cur))
@@ -572,7 +572,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
   const T dtdx = T(dt / geo.dx), dtdy = T(dt / geo.dy);
   const int nx = geo.nx, ny = geo.ny;
   const long long vs = geo.vstride;
-  const int i0 = blockIdx.x * TX, j0 = blockIdx.y * TY;
+  const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(nx + TX - 1) / TX;
+  const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
 
   // A: primitives and raw face fields on cells -2..TX+1 (ghosts through the boundary map;
   // a reflecting x pass negates IU and IA, a reflecting y pass IV and IB)
@@ -1085,7 +1086,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
       local = (s > local || !(s == s)) ? s : local;
     }
   }
-  block_max_to<NT>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x + blockIdx.y * gridDim.x), local, sred);
+  block_max_to<NT>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x), local, sred);
   if (first_block && tid < 64)
     step_end_bookkeeping(ctl, cur, dt);
 }

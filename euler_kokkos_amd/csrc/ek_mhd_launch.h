@@ -44,7 +44,7 @@ inline hipError_t launch_step(int rs, int st, const T* Uin, T* Uout, const Geom<
     default: f = pick<T, RS_HLLD>(st); break;
   }
   using M = M2Tile<T>;
-  dim3 grid((geo.nx + M::X - 1) / M::X, (geo.ny + M::Y - 1) / M::Y, 1);
+  dim3 grid((unsigned)((geo.nx + M::X - 1) / M::X) * (unsigned)((geo.ny + M::Y - 1) / M::Y));
   hipLaunchKernelGGL(f, grid, dim3(M::NT), 0, s, Uin, Uout, geo, gas, ctl);
   return hipGetLastError();
 }

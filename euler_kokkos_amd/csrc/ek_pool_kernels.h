@@ -14,7 +14,7 @@
 // each): 24 blasts of edges 64-320 took 57 us per step, 256 of edges 64-512 682 us (FP32), 100
 // of them 564 us (FP64) in a persistent grid walking ranges of the list. With 16 words per job
 // (4 to 64 measured alike but for 64's longer reads), one block per item and the items in
-// XCD order (pool_item): 30, 617 and 496 us. 3D jobs (six of edges 64-160): 452 -> 324 us
+// XCD order (33 us without it): 30, 617 and 496 us. 3D jobs (six of edges 64-160): 452 -> 324 us
 // FP32, 898 -> 709 us FP64.
 #pragma once
 
@@ -46,15 +46,6 @@ struct PoolWork {
   int tz_first; // z chunk * 2 + (1 if this item does the job's bookkeeping)
 };
 
-// Work item of this block: blocks are dealt to the 8 XCDs round robin, so each XCD gets a
-// contiguous eighth of the list and neighbouring tiles of a job share its L2 (33 -> 30 us for
-// the 24 blasts above; the remainder of the list keeps its order).
-__device__ __forceinline__ unsigned pool_item()
-{
-  const unsigned n8 = gridDim.x / 8, b = blockIdx.x;
-  return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;
-}
-
 template <class T, int TX, int TY, int NT, int RS, int ST>
 __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
@@ -62,7 +53,7 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  const PoolWork it = work[pool_item()];
+  const PoolWork it = work[xcd_order(blockIdx.x, gridDim.x)];
   const PoolJob<T> J = jobs[it.job];
   StepCtl ctl;
   ctl.ts = ts + J.slot0;
@@ -96,7 +87,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  const PoolWork it = work[pool_item()];
+  const PoolWork it = work[xcd_order(blockIdx.x, gridDim.x)];
   const PoolJob<T> J = jobs[it.job];
   StepCtl ctl;
   ctl.ts = ts + J.slot0;
