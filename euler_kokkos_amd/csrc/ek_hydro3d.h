@@ -464,12 +464,8 @@ __global__ __launch_bounds__(NT) void hydro3d_step(const T* __restrict__ Uin, T*
                                                    int ntx, int nty, int nchunk)
 {
   __shared__ double sred[NT / 64];
-  // XCD-aware tile order: blocks are dispatched round-robin over the 8 XCDs, so give each
-  // XCD a contiguous range of tiles (neighbours share halo lines in that XCD's L2).
-  const int nblk = ntx * nty * nchunk;
   const int b = blockIdx.x;
-  const int per = nblk / 8;
-  const int lb = (per * 8 == nblk) ? (b % 8) * per + b / 8 : b;
+  const int lb = (int)xcd_order((unsigned)b, gridDim.x);
   const int bx = lb % ntx, by = (lb / ntx) % nty, bz = lb / (ntx * nty);
   const bool first_block = b == 0;
   double dt;
