@@ -166,6 +166,15 @@ int ek::validate_params(const ek_params* p, std::string& why)
   return validate_common(p, why);
 }
 
+// z planes per block of the 3D hydro step
+static int z_chunk(const ek_params* p)
+{
+  if (p->dim != 3 || p->mhd)
+    return 1;
+  return p->precision == EK_FP64 ? ek::hydro3d_z_chunk<double>(p->nx, p->ny, p->nz)
+                                 : ek::hydro3d_z_chunk<float>(p->nx, p->ny, p->nz);
+}
+
 extern "C" int ek_create(const ek_params* params, ek_ctx** out)
 {
   if (!params || !out)
@@ -181,7 +190,7 @@ extern "C" int ek_create(const ek_params* params, ek_ctx** out)
   ek::fill_geom<double>(c->p, c->g64, c->gas64);
   ek::fill_geom<float>(c->p, c->g32, c->gas32);
   c->ncell = c->g64.vstride;
-  c->cz = params->dim == 3 ? ek::hydro3d_z_chunk(params->nx, params->ny, params->nz) : 1;
+  c->cz = z_chunk(params);
   hipError_t e;
   if ((e = hipGetDevice(&c->device)) != hipSuccess ||
       (e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess) {
@@ -706,7 +715,7 @@ extern "C" int ek_run_noalloc(const ek_params* params, void* U, void* U2, int ns
   ek::fill_geom<double>(c.p, c.g64, c.gas64);
   ek::fill_geom<float>(c.p, c.g32, c.gas32);
   c.ncell = c.g64.vstride;
-  c.cz = params->dim == 3 ? ek::hydro3d_z_chunk(params->nx, params->ny, params->nz) : 1;
+  c.cz = z_chunk(params);
   c.stream = (hipStream_t)stream;
   c.U[0] = U;
   c.U[1] = U2;

@@ -34,27 +34,42 @@ namespace ek {
 // Column tile of the single-grid 3D step: 16 x 8 cells, 256 threads.
 constexpr int T3X = 16, T3Y = 8, N3T = 256;
 
-// z-chunk length of the single-grid 3D step for an nx x ny x nz grid: the longest of 32,
-// 24, 16, 12, 8 that still gives 2048 blocks (8 per CU, enough to fill the 256 CUs with a
-// short tail), else 4. Each chunk re-traces two planes it does not update, so the longest
-// chunk that fills the GPU is fastest; on small grids shorter chunks are what fills it
-// (64^3: 0.134 ms per step at 32, 0.037 at 4; 192^3: 0.551 at 32, 0.532 at 24; 256^3 keeps 32).
-// The planes are then spread evenly over that many chunks: a step lasts as long as its
-// longest chunk (256^3: 1.20 ms at 32 planes, 1.25 at 30 or 34 and 1.33 at 36, whose last
-// chunk is short).
+// Blocks of the 3D step that 256 CUs hold at once: three per CU in FP64 (53.5 KB of LDS, 168
+// registers), five in FP32 (96 registers).
+template <class T>
+constexpr int T3SLOTS = 256 * (sizeof(T) == 8 ? 3 : 5);
+
+// z-chunk length of the single-grid 3D step for an nx x ny x nz grid. A block marches over its
+// chunk's planes and two more that it only traces, so long chunks do less work in all, but a
+// launch lasts as long as its last round of blocks. With n blocks on S slots a launch takes
+// about (chunk + a) * (floor(n / S) + b + (1 - b) frac) plane times, frac the part of S in an
+// incomplete last round (a block alone on its CU is faster per plane than one of three or
+// five): a, b fitted to 20 grids from 25x102x24 to 300x300x100 at every chunk length from 2 to
+// 64. The chunk with the smallest estimate is within 0.4 % of the fastest measured one on
+// average and 2.7 % at worst. (The longest chunk that gives 2048 blocks, the rule before it, is
+// 13 % off on average: 101x75x130 FP64 116 -> 95 us per step, FP32 54 -> 49; 128^3 174 -> 159 and
+// 80 -> 73; 32^3 24.7 -> 17.7; 256^3 unchanged.)
+template <class T>
 inline int hydro3d_z_chunk(int nx, int ny, int nz)
 {
+  constexpr double a = sizeof(T) == 8 ? 1.5 : 2.0, b = sizeof(T) == 8 ? 0.3 : 0.45;
   const long long tiles = (long long)((nx + T3X - 1) / T3X) * ((ny + T3Y - 1) / T3Y);
-  int cz = 4;
-  for (const int c : { 32, 24, 16, 12, 8 })
-    if (tiles * ((nz + c - 1) / c) >= 2048) {
-      cz = c;
+  int best = nz;
+  double least = 1e300;
+  for (int nch = 1; nch <= nz; nch++) {
+    const int cz = (nz + nch - 1) / nch;
+    if (cz > 64)
+      continue;
+    if (cz < 2)
       break;
+    const long long n = tiles * ((nz + cz - 1) / cz), rest = n % T3SLOTS<T>;
+    const double rounds = (double)(n / T3SLOTS<T>) + (rest ? b + (1.0 - b) * (double)rest / T3SLOTS<T> : 0.0);
+    if ((cz + a) * rounds < least) {
+      least = (cz + a) * rounds;
+      best = cz;
     }
-  if (cz >= nz)
-    return nz;
-  const int nch = (nz + cz - 1) / cz;
-  return (nz + nch - 1) / nch;
+  }
+  return best;
 }
 
 template <int TX, int TY, int NT>
