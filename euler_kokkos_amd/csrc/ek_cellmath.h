@@ -174,13 +174,13 @@ __device__ __forceinline__ void prims(const Gas<T>& g, const T* u, T* q)
     // FP32 state: when the internal energy is a small remainder of E/rho (more than 7 of
     // the 24 mantissa bits cancelled), recover it in FP64 from the same conserved values.
     if (e < T(0.0078125) * et) {
-      const double rd = inv_of((double)d).y, ix = (double)u[IU] * rd, iy = (double)u[IV] * rd;
+      const double dd = d, ix = (double)u[IU] / dd, iy = (double)u[IV] / dd;
       double ek = ix * ix + iy * iy;
       if constexpr (DIM == 3) {
-        const double iz = (double)u[IW] * rd;
+        const double iz = (double)u[IW] / dd;
         ek += iz * iz;
       }
-      e = (T)((double)u[IP] * rd - 0.5 * ek);
+      e = (T)((double)u[IP] / dd - 0.5 * ek);
     }
   }
   q[ID] = d;

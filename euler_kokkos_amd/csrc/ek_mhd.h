@@ -49,12 +49,11 @@ __device__ __forceinline__ void constoprim(const Gas<T>& g, const T* u, T mx, T 
     // FP32 state: p = (gamma-1)(E - rho v^2/2 - B^2/2) recovered in FP64 where more than 7
     // of the 24 mantissa bits cancel
     if (eint < T(0.0078125) * quot(u[IP], id)) {
-      const double rd = inv_of((double)q[ID]).y;
-      const double ux = (double)u[IU] * rd, uy = (double)u[IV] * rd, uz = (double)u[IW] * rd;
+      const double d = q[ID], ux = (double)u[IU] / d, uy = (double)u[IV] / d, uz = (double)u[IW] / d;
       const double bx = 0.5 * ((double)u[IA] + (double)mx), by = 0.5 * ((double)u[IB] + (double)my),
                    bz = 0.5 * ((double)u[IC] + (double)mz);
       const double em = 0.5 * (bx * bx + by * by + bz * bz);
-      eint = (T)(((double)u[IP] - em) * rd - 0.5 * (ux * ux + uy * uy + uz * uz));
+      eint = (T)(((double)u[IP] - em) / d - 0.5 * (ux * ux + uy * uy + uz * uz));
     }
   }
   q[IP] = emax(g.gm1 * q[ID] * eint, q[ID] * g.smallp);
