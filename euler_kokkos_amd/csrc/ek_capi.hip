@@ -720,7 +720,7 @@ extern "C" int ek_run_noalloc(const ek_params* params, void* U, void* U2, int ns
   c.U[0] = U;
   c.U[1] = U2;
   if (c.p.mhd && c.p.dim == 3) {
-    const long long wb = ek::fp64::mhd3_scratch_elems(c.p.nx, c.p.ny, c.p.nz) * (long long)c.elem;
+    const long long wb = ek::mhd3_limit_elems(c.p) * (long long)c.elem;
     if ((double)wb > (double)(kScratchBytes - kScratchWork))
       return fail(nullptr, EK_EINVAL,
                   "grid too large for ek_run_noalloc: the 3D MHD work area needs " + std::to_string(wb) +

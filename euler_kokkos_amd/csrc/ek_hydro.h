@@ -221,6 +221,32 @@ __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
   return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;
 }
 
+// Planes per z-chunk of a launch of `tiles` column tiles over n planes: a block marches over its
+// chunk, so long chunks repeat less work at their ends, but a launch lasts as long as its last
+// round of blocks. With m blocks on `slots` places a launch takes about (chunk + a) *
+// (floor(m / slots) + b + (1 - b) frac) plane times, frac the part of the places an incomplete
+// last round fills (a block alone on its CU is faster per plane than one of several). Returns
+// the chunk length between lo and hi with the smallest estimate.
+inline int z_chunk_of(long long tiles, int n, int slots, double a, double b, int lo, int hi)
+{
+  int best = n < hi ? n : hi;
+  double least = 1e300;
+  for (int nch = 1; nch <= n; nch++) {
+    const int cz = (n + nch - 1) / nch;
+    if (cz > hi)
+      continue;
+    if (cz < lo)
+      break;
+    const long long m = tiles * ((n + cz - 1) / cz), rest = m % slots;
+    const double rounds = (double)(m / slots) + (rest ? b + (1.0 - b) * (double)rest / slots : 0.0);
+    if ((cz + a) * rounds < least) {
+      least = (cz + a) * rounds;
+      best = cz;
+    }
+  }
+  return best;
+}
+
 // Block max then one atomic per block. NaN (a failed cell) wins: its bit pattern is above
 // every finite double's, so a blown-up state yields dt = NaN instead of being skipped.
 template <int NT>

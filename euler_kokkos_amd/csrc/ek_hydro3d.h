@@ -39,37 +39,17 @@ constexpr int T3X = 16, T3Y = 8, N3T = 256;
 template <class T>
 constexpr int T3SLOTS = 256 * (sizeof(T) == 8 ? 3 : 5);
 
-// z-chunk length of the single-grid 3D step for an nx x ny x nz grid. A block marches over its
-// chunk's planes and two more that it only traces, so long chunks do less work in all, but a
-// launch lasts as long as its last round of blocks. With n blocks on S slots a launch takes
-// about (chunk + a) * (floor(n / S) + b + (1 - b) frac) plane times, frac the part of S in an
-// incomplete last round (a block alone on its CU is faster per plane than one of three or
-// five): a, b fitted to 20 grids from 25x102x24 to 300x300x100 at every chunk length from 2 to
-// 64. The chunk with the smallest estimate is within 0.4 % of the fastest measured one on
-// average and 2.7 % at worst. (The longest chunk that gives 2048 blocks, the rule before it, is
-// 13 % off on average: 101x75x130 FP64 116 -> 95 us per step, FP32 54 -> 49; 128^3 174 -> 159 and
-// 80 -> 73; 32^3 24.7 -> 17.7; 256^3 unchanged.)
+// z-chunk length of the single-grid 3D step for an nx x ny x nz grid: z_chunk_of with a, b
+// fitted to 20 grids from 25x102x24 to 300x300x100 at every chunk length from 2 to 64. The
+// chunk it picks is within 0.4 % of the fastest measured one on average and 2.7 % at worst.
+// (The longest chunk that gives 2048 blocks, the rule before it, is 13 % off on average:
+// 101x75x130 FP64 116 -> 95 us per step, FP32 54 -> 49; 128^3 174 -> 159 and 80 -> 73; 32^3 24.7
+// -> 17.7; 256^3 unchanged.)
 template <class T>
 inline int hydro3d_z_chunk(int nx, int ny, int nz)
 {
-  constexpr double a = sizeof(T) == 8 ? 1.5 : 2.0, b = sizeof(T) == 8 ? 0.3 : 0.45;
   const long long tiles = (long long)((nx + T3X - 1) / T3X) * ((ny + T3Y - 1) / T3Y);
-  int best = nz;
-  double least = 1e300;
-  for (int nch = 1; nch <= nz; nch++) {
-    const int cz = (nz + nch - 1) / nch;
-    if (cz > 64)
-      continue;
-    if (cz < 2)
-      break;
-    const long long n = tiles * ((nz + cz - 1) / cz), rest = n % T3SLOTS<T>;
-    const double rounds = (double)(n / T3SLOTS<T>) + (rest ? b + (1.0 - b) * (double)rest / T3SLOTS<T> : 0.0);
-    if ((cz + a) * rounds < least) {
-      least = (cz + a) * rounds;
-      best = cz;
-    }
-  }
-  return best;
+  return z_chunk_of(tiles, nz, T3SLOTS<T>, sizeof(T) == 8 ? 1.5 : 2.0, sizeof(T) == 8 ? 0.3 : 0.45, 2, 64);
 }
 
 template <int TX, int TY, int NT>

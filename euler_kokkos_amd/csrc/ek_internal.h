@@ -14,6 +14,14 @@ namespace ek {
 template <class T>
 struct PoolJobM;  // 3D MHD job record of the job pool (ek_pool_mhd3d.h)
 
+// Work reals per ghost-padded cell that the limits of ek_run_noalloc and the job pool count for
+// 3D MHD (include/ek_hip.h, include/ek_pool.h); the pipeline itself uses mhd3_scratch_elems.
+constexpr int kMhd3LimitReals = 78;
+inline long long mhd3_limit_elems(const ek_params& p)
+{
+  return (long long)kMhd3LimitReals * (p.nx + 6) * (p.ny + 6) * (long long)(p.nz + 6);
+}
+
 // Checks an ek_params against what this library provides (ek_capi.hip); 0 when valid.
 int validate_params(const ek_params* p, std::string& why);
 // FP32 copy of n FP64 values already on the device (round to nearest, denormals kept, as
@@ -53,12 +61,13 @@ hipError_t mhd3_inv_dt(const double* U, const Geom<double>& geo, const Gas<doubl
                        unsigned long long* spread, int nspread,
                   hipStream_t s);
 long long mhd3_scratch_elems(int nx, int ny, int nz);
-// 3D MHD jobs of the job pool (ek_mhd3d_fp64.hip): the five pipeline kernels over the work
-// lists wp (padded-grid chunks) and wu (interior chunks); grid[5] from pool_mhd3_grids
+// 3D MHD jobs of the job pool (ek_mhd3d_fp64.hip): the four pipeline kernels over the work
+// lists wp (padded-grid chunks), wf (column tiles of the flux/EMF kernel) and wu (interior
+// chunks); ugrid from pool_mhd3_update_grid
 hipError_t pool_mhd3_step(int rs, int st, const double* Ua, double* Ub, double* W, const PoolJobM<double>* jobs,
-                          const PoolWork* wp, int np, const PoolWork* wu, int nu, TimeSlot* ts, int slot,
-                          const int* grid, hipStream_t s);
-void pool_mhd3_grids(int rs, int st, int cus, int* grid);
+                          const PoolWork* wp, int np, const PoolWork* wf, int nf, const PoolWork* wu, int nu,
+                          TimeSlot* ts, int slot, int ugrid, hipStream_t s);
+int pool_mhd3_update_grid(int cus);
 } // namespace fp64
 namespace fp32 {
 hipError_t step(int dim, int rs, int st, const float* Uin, float* Uout, const Geom<float>& geo,
@@ -89,11 +98,12 @@ hipError_t mhd3_inv_dt(const float* U, const Geom<float>& geo, const Gas<float>&
                        unsigned long long* spread, int nspread,
                   hipStream_t s);
 long long mhd3_scratch_elems(int nx, int ny, int nz);
-// 3D MHD jobs of the job pool (ek_mhd3d_fp32.hip): the five pipeline kernels over the work
-// lists wp (padded-grid chunks) and wu (interior chunks); grid[5] from pool_mhd3_grids
+// 3D MHD jobs of the job pool (ek_mhd3d_fp32.hip): the four pipeline kernels over the work
+// lists wp (padded-grid chunks), wf (column tiles of the flux/EMF kernel) and wu (interior
+// chunks); ugrid from pool_mhd3_update_grid
 hipError_t pool_mhd3_step(int rs, int st, const float* Ua, float* Ub, float* W, const PoolJobM<float>* jobs,
-                          const PoolWork* wp, int np, const PoolWork* wu, int nu, TimeSlot* ts, int slot,
-                          const int* grid, hipStream_t s);
-void pool_mhd3_grids(int rs, int st, int cus, int* grid);
+                          const PoolWork* wp, int np, const PoolWork* wf, int nf, const PoolWork* wu, int nu,
+                          TimeSlot* ts, int slot, int ugrid, hipStream_t s);
+int pool_mhd3_update_grid(int cus);
 } // namespace fp32
 } // namespace ek

@@ -377,6 +377,14 @@ __device__ __forceinline__ void fast_xy(const Gas<T>& g, const Edge<T>& s, T& fx
   fy = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * s.b * s.b, ir)));
 }
 
+// u b - v a. In FP32 the first product fuses, whatever the block the compiler puts the
+// difference in.
+__device__ __forceinline__ double crossed(double u, double b, double v, double a) { return u * b - v * a; }
+__device__ __forceinline__ float crossed(float u, float b, float v, float a)
+{
+  return __builtin_fmaf(u, b, -(v * a));
+}
+
 // compute_emf<EMFZ> + mag_riemann2d_hlld (RiemannSolvers_MHD.h:395-627, 648-871). The
 // edge states arrive as the trace produced them (qRT, qRB, qLT, qLB); the solver's
 // LL/RL/LR/RR states are RT/LT/RB/LB with the transverse face fields averaged.
@@ -391,10 +399,10 @@ __device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
   const T bR = T(0.5) * (LT.b + LB.b);
   LL.a = aT; RL.a = aT; LR.a = aB; RR.a = aB;
   LL.b = bL; RL.b = bR; LR.b = bL; RR.b = bR;
-  const T ELL = LL.u * LL.b - LL.v * LL.a;
-  const T ERL = RL.u * RL.b - RL.v * RL.a;
-  const T ELR = LR.u * LR.b - LR.v * LR.a;
-  const T ERR = RR.u * RR.b - RR.v * RR.a;
+  const T ELL = crossed(LL.u, LL.b, LL.v, LL.a);
+  const T ERL = crossed(RL.u, RL.b, RL.v, RL.a);
+  const T ELR = crossed(LR.u, LR.b, LR.v, LR.a);
+  const T ERR = crossed(RR.u, RR.b, RR.v, RR.a);
   const T rLL = LL.r, uLL = LL.u, vLL = LL.v, aLL = LL.a, bLL = LL.b, cLL = LL.c, pLL = LL.p;
   const T rLR = LR.r, uLR = LR.u, vLR = LR.v, aLR = LR.a, bLR = LR.b, cLR = LR.c, pLR = LR.p;
   const T rRL = RL.r, uRL = RL.u, vRL = RL.v, aRL = RL.a, bRL = RL.b, cRL = RL.c, pRL = RL.p;
@@ -481,7 +489,17 @@ __device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
   tmpE = quot_any(quot_any(SAL * SAB * EstarRR - SAL * SAT * EstarRL - SAR * SAB * EstarLR + SAR * SAT * EstarLL, iw),
                   ih) -
          quot(SAT * SAB, ih) * (AstarT - AstarB) + quot(SAR * SAL, iw) * (BstarR - BstarL);
-  E += on(!Bp && Tp && !Lp && Rp) * tmpE;
+  const bool middle = !Bp && Tp && !Lp && Rp;
+  E += on(middle) * tmpE;
+  // Subsonic in both directions, with a finite candidate: the other four count zero times (they
+  // are finite too: short of overflow their terms are the same products). A wave all of whose
+  // lanes are leaves here, without the last fifth of the solve (2D MHD 1024^2 207 -> 204 us per
+  // step, 3D MHD 128^3 983 -> 975). Not in FP32, where splitting the solve would change
+  // which of its products are fused.
+  if constexpr (sizeof(T) == 8) {
+    if (middle && __builtin_isfinite(tmpE))
+      return E;
+  }
   tmpE = quot_any(SAR * EstarLLx - SAL * EstarRLx + SAR * SAL * (bRL - bLL), iw);
   tmpE = on(Lp) * ELL + on(!Lp && !Rp) * ERL + on(!Lp && Rp) * tmpE;
   E += on(Bp) * tmpE;

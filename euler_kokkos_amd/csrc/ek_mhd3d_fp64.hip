@@ -14,10 +14,10 @@ static hipError_t launch3(const double* Uin, double* Uout, double* S, const mhd3
   const long long nu = (geo.vstride + 255) / 256;
   const unsigned ni = (unsigned)(nu < mhd3::MHD3_UPDATE_BLOCKS ? nu : mhd3::MHD3_UPDATE_BLOCKS);
   hipLaunchKernelGGL(mhd3::padprims_kernel<double>, dim3(nb), dim3(256), 0, s, Uin, S, w, geo, gas, ctl);
-  hipLaunchKernelGGL((mhd3::efield_kernel<double, ST>), dim3(nb), dim3(256), 0, s, S, w, ctl);
-  hipLaunchKernelGGL((mhd3::trace_kernel<double, ST>), dim3(nb), dim3(256), 0, s, S, w, geo, gas, ctl);
-  const unsigned nfe = 32u * ((nb + 7u) / 8u); // 4 tasks per chunk, chunks in groups of 8
-  hipLaunchKernelGGL((mhd3::fluxemf_kernel<double, RS>), dim3(nfe), dim3(256), 0, s, S, w, gas, ctl);
+  hipLaunchKernelGGL(mhd3::efield_kernel<double>, dim3(nb), dim3(256), 0, s, S, w, ctl);
+  const mhd3::FluxGrid fg = mhd3::flux_grid(geo);
+  hipLaunchKernelGGL((mhd3::fluxemf_kernel<double, RS, ST>), dim3(fg.ntx * fg.nty * fg.ntz), dim3(mhd3::FCN), 0, s, S, w, geo,
+                     gas, ctl, fg.cz, fg.ntx, fg.nty);
   hipLaunchKernelGGL(mhd3::update_kernel<double>, dim3(ni), dim3(256), 0, s, S, Uout, w, geo, gas, ctl);
   return hipGetLastError();
 }
@@ -61,15 +61,15 @@ long long mhd3_scratch_elems(int nx, int ny, int nz)
 }
 
 hipError_t pool_mhd3_step(int rs, int st, const double* Ua, double* Ub, double* W, const PoolJobM<double>* jobs,
-                          const PoolWork* wp, int np, const PoolWork* wu, int nu, TimeSlot* ts, int slot,
-                          const int* grid, hipStream_t s)
+                          const PoolWork* wp, int np, const PoolWork* wf, int nf, const PoolWork* wu, int nu,
+                          TimeSlot* ts, int slot, int ugrid, hipStream_t s)
 {
-  return pool::mhd3_step<double>(rs, st, Ua, Ub, W, jobs, wp, np, wu, nu, ts, slot, grid, s);
+  return pool::mhd3_step<double>(rs, st, Ua, Ub, W, jobs, wp, np, wf, nf, wu, nu, ts, slot, ugrid, s);
 }
 
-void pool_mhd3_grids(int rs, int st, int cus, int* grid)
+int pool_mhd3_update_grid(int cus)
 {
-  pool::mhd3_grids_for<double>(rs, st, cus, grid);
+  return pool::mhd3_update_grid<double>(cus);
 }
 
 } // namespace fp64

@@ -88,7 +88,10 @@ struct ek_pool {
   ek::PoolWork* dworkU = nullptr;
   int nworkU = 0;
   int workU_cap = 0;
-  int mgrid[5] = { 1, 1, 1, 1, 1 };
+  ek::PoolWork* dworkF = nullptr; // flux/EMF column tiles
+  int nworkF = 0;
+  int workF_cap = 0;
+  int ugrid = 1; // blocks of the update kernel
   int test_fail_admit = 0; // ek_pool_test_fail_admit: 0 off, else the admission step that fails
   // asynchronous admission: uploads (and the FP32 rounding) run on their own stream, with
   // their own staging buffer, one completion event per job slot
@@ -164,6 +167,21 @@ static ek::PoolJob<T> make_record(const ek_pool* p, int id)
   return r;
 }
 
+// column tiles and z-chunks of a 3D MHD job's flux/EMF items
+static ek::mhd3::FluxGrid flux_grid_of(const ek_pool* p, const ek_params& j)
+{
+  if (p->fp64) {
+    ek::Geom<double> g;
+    ek::Gas<double> gs;
+    ek::fill_geom<double>(j, g, gs);
+    return ek::mhd3::flux_grid(g);
+  }
+  ek::Geom<float> g;
+  ek::Gas<float> gs;
+  ek::fill_geom<float>(j, g, gs);
+  return ek::mhd3::flux_grid(g);
+}
+
 // 3D MHD record of job `id`
 template <class T>
 static ek::PoolJobM<T> make_record_m(const ek_pool* p, int id)
@@ -183,6 +201,7 @@ static ek::PoolJobM<T> make_record_m(const ek_pool* p, int id)
   r.w.PY = h.p.ny + 6;
   r.w.PZ = h.p.nz + 6;
   r.w.PN = (long long)r.w.PX * r.w.PY * r.w.PZ;
+  r.cz = flux_grid_of(p, h.p).cz;
   ek::fill_geom<T>(h.p, r.geo, r.gas);
   return r;
 }
@@ -251,12 +270,12 @@ static int put_list(ek_pool* p, const std::vector<ek::PoolWork>& w, ek::PoolWork
   return EK_OK;
 }
 
-// 3D MHD work lists: (job, 256-cell chunk of its padded grid) for the four padded-grid
-// kernels, (job, 4096-cell chunk of its interior) for the update, the job's first chunk
-// flagged for its time bookkeeping
+// 3D MHD work lists: (job, 4096-cell chunk of its padded grid) for the two padded-grid
+// kernels, (job, column tile, z-chunk) for the flux/EMF kernel, (job, 4096-cell chunk of its
+// interior) for the update, the job's first chunk flagged for its time bookkeeping
 static int rebuild_work_mhd3(ek_pool* p)
 {
-  std::vector<ek::PoolWork> wp, wu;
+  std::vector<ek::PoolWork> wp, wf, wu;
   for (int id = 0; id < (int)p->jobs.size(); id++) {
     const HostJob& h = p->jobs[id];
     if (!h.used || h.finished || h.pending)
@@ -265,14 +284,22 @@ static int rebuild_work_mhd3(ek_pool* p)
     const long long np = (pn + ek::MP_CHUNK - 1) / ek::MP_CHUNK, nu = (h.ncell + ek::MU_CHUNK - 1) / ek::MU_CHUNK;
     for (long long c = 0; c < np; c++)
       wp.push_back(ek::PoolWork{ id, (int)c, 0, 0 });
+    const ek::mhd3::FluxGrid fg = flux_grid_of(p, h.p);
+    for (int tz = 0; tz < fg.ntz; tz++)
+      for (int ty = 0; ty < fg.nty; ty++)
+        for (int tx = 0; tx < fg.ntx; tx++)
+          wf.push_back(ek::PoolWork{ id, tx, ty, tz });
     for (long long c = 0; c < nu; c++)
       wu.push_back(ek::PoolWork{ id, (int)c, 0, c == 0 ? 1 : 0 });
   }
   if (int rc = put_list(p, wp, &p->dwork, &p->work_cap))
     return rc;
+  if (int rc = put_list(p, wf, &p->dworkF, &p->workF_cap))
+    return rc;
   if (int rc = put_list(p, wu, &p->dworkU, &p->workU_cap))
     return rc;
   p->nwork = (int)wp.size();
+  p->nworkF = (int)wf.size();
   p->nworkU = (int)wu.size();
   p->graph_ok = false;
   return EK_OK;
@@ -314,13 +341,8 @@ static int rebuild_work(ek_pool* p)
 
 static void set_grid(ek_pool* p)
 {
-  if (p->mhd3) {
-    const int rs = p->kind.riemann, st = (int)p->kind.slope_type;
-    if (p->fp64)
-      ek::fp64::pool_mhd3_grids(rs, st, p->cus, p->mgrid);
-    else
-      ek::fp32::pool_mhd3_grids(rs, st, p->cus, p->mgrid);
-  }
+  if (p->mhd3)
+    p->ugrid = p->fp64 ? ek::fp64::pool_mhd3_update_grid(p->cus) : ek::fp32::pool_mhd3_update_grid(p->cus);
 }
 
 static hipError_t launch_one(ek_pool* p, long long n)
@@ -331,11 +353,11 @@ static hipError_t launch_one(ek_pool* p, long long n)
     const int rs = p->kind.riemann;
     if (p->fp64)
       return ek::fp64::pool_mhd3_step(rs, st, (const double*)p->A[par], (double*)p->A[1 - par], (double*)p->W,
-                                      (const ek::PoolJobM<double>*)p->djobs, p->dwork, p->nwork, p->dworkU,
-                                      p->nworkU, p->ts, slot, p->mgrid, p->stream);
+                                      (const ek::PoolJobM<double>*)p->djobs, p->dwork, p->nwork, p->dworkF, p->nworkF,
+                                      p->dworkU, p->nworkU, p->ts, slot, p->ugrid, p->stream);
     return ek::fp32::pool_mhd3_step(rs, st, (const float*)p->A[par], (float*)p->A[1 - par], (float*)p->W,
-                                    (const ek::PoolJobM<float>*)p->djobs, p->dwork, p->nwork, p->dworkU, p->nworkU,
-                                    p->ts, slot, p->mgrid, p->stream);
+                                    (const ek::PoolJobM<float>*)p->djobs, p->dwork, p->nwork, p->dworkF, p->nworkF,
+                                    p->dworkU, p->nworkU, p->ts, slot, p->ugrid, p->stream);
   }
   if (p->fp64)
     return ek::fp64::pool_step(kind_dim(p), p->variant, st, (const double*)p->A[par], (double*)p->A[1 - par],
@@ -441,7 +463,7 @@ static void arena_free(ek_pool* p, long long off, long long n)
 // elements of a 3D MHD job's padded work area
 static long long work_elems(const ek_params& j)
 {
-  return ek::fp64::mhd3_scratch_elems(j.nx, j.ny, j.nz);
+  return ek::mhd3_limit_elems(j);
 }
 
 static int ensure_stage(ek_pool* p, long long n)
@@ -546,6 +568,7 @@ extern "C" void ek_pool_destroy(ek_pool* p)
   hipFree(p->djobs);
   hipFree(p->spread);
   hipFree(p->dwork);
+  hipFree(p->dworkF);
   hipFree(p->dworkU);
   hipFree(p->W);
   hipFree(p->stage);

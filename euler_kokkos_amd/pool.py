@@ -2,7 +2,7 @@
 
 A :class:`Pool` keeps many independent grids (hydro 2D/3D, or 3D MHD) resident in one
 device arena and advances all unfinished jobs by one step of their own dt per pool step (one
-kernel over a (job, tile) work list for hydro, the five 3D MHD pipeline kernels
+kernel over a (job, tile) work list for hydro, the four 3D MHD pipeline kernels
 each over all jobs' chunks for MHD, replayed from a captured HIP graph). A job's result
 equals its single-grid :class:`native.Context` run.
 

@@ -5,7 +5,7 @@ Jobs arrive on a seeded Poisson process. Each job kind has its own pool and its 
 the loops running side by side: at every turn a loop admits, in arrival order, each job of
 its kind that has arrived and fits in the pool's memory (its upload runs on the pool's upload
 stream beside the steps, and it joins the first step after the upload); then it advances all admitted jobs
-of the pool together (one launch per step for a hydro pool, the five 3D MHD
+of the pool together (one launch per step for a hydro pool, the four 3D MHD
 kernels each over all jobs for an MHD pool, replayed from a captured graph); finished jobs
 are collected and retired, which frees memory for the queue. Time-to-solution is measured
 from a job's arrival to its completion; throughput over the whole stream.

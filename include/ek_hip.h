@@ -119,7 +119,7 @@ int ek_run(ek_ctx* ctx, int nsteps, int nStepmax, double tEnd, double* t_io, int
  * that stream to read the final time. The time slots, CFL words and, for 3D MHD, the padded
  * work area live in a fixed device array of EK_NOALLOC_SCRATCH_BYTES per device, held from
  * the library's first use on that device until the process ends: a 3D MHD grid whose work
- * area (78 reals per ghost-padded cell) does not fit is rejected with EK_EINVAL. Every call
+ * area, counted as 78 reals per ghost-padded cell, does not fit is rejected with EK_EINVAL. Every call
  * on one device uses the same array, so calls that overlap on one device race; each call
  * clears what it needs first. Errors are reported through ek_last_error(NULL). */
 int ek_run_noalloc(const ek_params* params, void* U, void* U2, int nsteps, int nStepmax, double tEnd,

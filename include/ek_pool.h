@@ -14,7 +14,7 @@
  * list; consecutive steps over an unchanged job set are replayed from a
  * captured HIP graph. Tile shapes are chosen by ek_pool_autotune. A 3D MHD pool also keeps
  * each job's ghost-padded work area (78 reals per padded cell) in a work buffer that takes
- * 84 % of arena_bytes (the two state buffers take the rest), and one pool step is the five
+ * 84 % of arena_bytes (the two state buffers take the rest), and one pool step is the four
  * kernels of the 3D MHD step, each over all active jobs.
  *
  * All calls return 0 or an EK_E* code (include/ek_hip.h) with a message from
