@@ -332,10 +332,12 @@ __device__ __forceinline__ void hllc(const Gas<T>& g, const T* ql, const T* qr, 
   if constexpr (NV == 5)
     ecinr += h * rr * qr[IW] * qr[IW];
   const T etotr = pr * g.entho + ecinr;
-  const T cfastl = esqrt(emax(quot(g.gamma0 * pl, inv_of(rl)), g.smallc2));
-  const T cfastr = esqrt(emax(quot(g.gamma0 * pr, inv_of(rr)), g.smallc2));
-  const T SL = emin(ul, ur) - emax(cfastl, cfastr);
-  const T SR = emax(ul, ur) + emax(cfastl, cfastr);
+  // the faster of the two sound speeds (emax(sqrt(x), sqrt(y)) is sqrt(emax(x, y)): a root is
+  // monotone, FP32's over every float too)
+  const T cfast = esqrt(emax(emax(quot(g.gamma0 * pl, inv_of(rl)), g.smallc2),
+                             emax(quot(g.gamma0 * pr, inv_of(rr)), g.smallc2)));
+  const T SL = emin(ul, ur) - cfast;
+  const T SR = emax(ul, ur) + cfast;
   const T rcl = rl * (ul - SL);
   const T rcr = rr * (SR - ur);
   const Inv<T> irc = inv_of(rcr + rcl);

@@ -59,9 +59,11 @@ __device__ __forceinline__ void constoprim(const Gas<T>& g, const T* u, T mx, T 
   q[IP] = emax(g.gm1 * q[ID] * eint, q[ID] * g.smallp);
 }
 
-// find_speed_fast<dir> (src/shared/mhd_utils.h:89-117)
+// Square of find_speed_fast<dir> (src/shared/mhd_utils.h:89-117). The solvers only want the
+// largest of several speeds, and take one root of the largest square: the same value, since a
+// root is monotone (FP32's over every float too), and a NaN passes through the same comparisons.
 template <class T, int DIR>
-__device__ __forceinline__ T speed_fast(const Gas<T>& g, const T* q)
+__device__ __forceinline__ T speed_fast2(const Gas<T>& g, const T* q)
 {
   const T d = q[ID], p = q[IP], a = q[IA], b = q[IB], c = q[IC];
   const T b2 = a * a + b * b + c * c;
@@ -69,7 +71,13 @@ __device__ __forceinline__ T speed_fast(const Gas<T>& g, const T* q)
   const T c2 = quot(g.gamma0 * p, id);
   const T d2 = T(0.5) * (quot(b2, id) + c2);
   const T n = DIR == 0 ? a : (DIR == 1 ? b : c);
-  return esqrt(d2 + esqrt(d2 * d2 - quot(c2 * n * n, id)));
+  return d2 + esqrt(d2 * d2 - quot(c2 * n * n, id));
+}
+
+template <class T, int DIR>
+__device__ __forceinline__ T speed_fast(const Gas<T>& g, const T* q)
+{
+  return esqrt(speed_fast2<T, DIR>(g, q));
 }
 
 // find_speed_info<TWO_D> (mhd_utils.h:319-366) folded into ComputeDtFunctor2D_MHD
@@ -170,9 +178,9 @@ __device__ __forceinline__ void hll(const Gas<T>& g, T* ql, T* qr, T* flux)
   T ul[NV], fl[NV], ur[NV], fr[NV];
   mhd_flux(g, ql, ul, fl);
   mhd_flux(g, qr, ur, fr);
-  const T cfl = speed_fast<T, 0>(g, ql), cfr = speed_fast<T, 0>(g, qr);
-  const T sl = emin(emin(ql[IU], qr[IU]) - emax(cfl, cfr), T(0));
-  const T sr = emax(emax(ql[IU], qr[IU]) + emax(cfl, cfr), T(0));
+  const T cf = esqrt(emax(speed_fast2<T, 0>(g, ql), speed_fast2<T, 0>(g, qr)));
+  const T sl = emin(emin(ql[IU], qr[IU]) - cf, T(0));
+  const T sr = emax(emax(ql[IU], qr[IU]) + cf, T(0));
   const Inv<T> iw = inv_of(sr - sl);
 #pragma unroll
   for (int n = 0; n < NV; n++)
@@ -223,11 +231,11 @@ __device__ __forceinline__ void hlld(const Gas<T>& g, const T* qleft, const T* q
   const T vdotbr = ur * a + vr * br + wr * cr;
   T qtmp[NV];
   qtmp[ID] = rl; qtmp[IP] = pl; qtmp[IA] = a; qtmp[IB] = bl; qtmp[IC] = cl;
-  const T cfastl = speed_fast<T, 0>(g, qtmp);
+  const T cfastl2 = speed_fast2<T, 0>(g, qtmp);
   qtmp[ID] = rr; qtmp[IP] = pr; qtmp[IB] = br; qtmp[IC] = cr;
-  const T cfastr = speed_fast<T, 0>(g, qtmp);
-  const T sl = emin(ul, ur) - emax(cfastl, cfastr);
-  const T sr = emax(ul, ur) + emax(cfastl, cfastr);
+  const T cfast = esqrt(emax(cfastl2, speed_fast2<T, 0>(g, qtmp)));
+  const T sl = emin(ul, ur) - cfast;
+  const T sr = emax(ul, ur) + cfast;
   const T rcl = rl * (ul - sl);
   const T rcr = rr * (sr - ur);
   const Inv<T> irc = inv_of(rcr + plain(rcl)); // FP32: only rcr's product fuses into the sum
@@ -365,16 +373,16 @@ struct Edge {
   T r, p, u, v, a, b, c;
 };
 
-// find_speed_fast along both directions of the edge plane (src/shared/mhd_utils.h:89-117)
+// squares of find_speed_fast along both directions of the edge plane (src/shared/mhd_utils.h:89-117)
 template <class T>
-__device__ __forceinline__ void fast_xy(const Gas<T>& g, const Edge<T>& s, T& fx, T& fy)
+__device__ __forceinline__ void fast2_xy(const Gas<T>& g, const Edge<T>& s, T& fx, T& fy)
 {
   const T b2 = s.a * s.a + s.b * s.b + s.c * s.c;
   const Inv<T> ir = inv_of(s.r);
   const T c2 = quot(g.gamma0 * s.p, ir);
   const T d2 = T(0.5) * (quot(b2, ir) + c2);
-  fx = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * s.a * s.a, ir)));
-  fy = esqrt(d2 + esqrt(d2 * d2 - quot(c2 * s.b * s.b, ir)));
+  fx = d2 + esqrt(d2 * d2 - quot(c2 * s.a * s.a, ir));
+  fy = d2 + esqrt(d2 * d2 - quot(c2 * s.b * s.b, ir));
 }
 
 // u b - v a. In FP32 the first product fuses, whatever the block the compiler puts the
@@ -408,11 +416,11 @@ __device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
   const T rRL = RL.r, uRL = RL.u, vRL = RL.v, aRL = RL.a, bRL = RL.b, cRL = RL.c, pRL = RL.p;
   const T rRR = RR.r, uRR = RR.u, vRR = RR.v, aRR = RR.a, bRR = RR.b, cRR = RR.c, pRR = RR.p;
   T fxLL, fxLR, fxRL, fxRR, fyLL, fyLR, fyRL, fyRR;
-  fast_xy(g, LL, fxLL, fyLL);
-  fast_xy(g, LR, fxLR, fyLR);
-  fast_xy(g, RL, fxRL, fyRL);
-  fast_xy(g, RR, fxRR, fyRR);
-  const T fx = fmax4(fxLL, fxLR, fxRL, fxRR), fy = fmax4(fyLL, fyLR, fyRL, fyRR);
+  fast2_xy(g, LL, fxLL, fyLL);
+  fast2_xy(g, LR, fxLR, fyLR);
+  fast2_xy(g, RL, fxRL, fyRL);
+  fast2_xy(g, RR, fxRR, fyRR);
+  const T fx = esqrt(fmax4(fxLL, fxLR, fxRL, fxRR)), fy = esqrt(fmax4(fyLL, fyLR, fyRL, fyRR));
   const T SL = fmin4(uLL, uLR, uRL, uRR) - fx;
   const T SR = fmax4(uLL, uLR, uRL, uRR) + fx;
   const T SB = fmin4(vLL, vLR, vRL, vRR) - fy;
