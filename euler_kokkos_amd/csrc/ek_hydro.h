@@ -352,52 +352,99 @@ __device__ __forceinline__ double cfl_term(const Gas<T>& gas, const T* u, const 
 // positions, slopes+trace on the tile and its 1-wide halo cross, (TX+1)*TY x-faces and
 // TX*(TY+1) y-faces, then the update of the TX*TY cells. Every face flux is solved once
 // per tile; slopes are computed once per position (the reference recomputes them up to 3x).
+//
+// FP64 issue is the bound of a large grid (65 % VALU busy at 16x16 with primitives and face
+// states side by side in 47.6 KB of LDS: three blocks per CU); latency is that of a small one
+// (loads, four barriers, a chain of divisions and roots per phase). So
+// - CMP: one traced cell per thread, its face states kept in registers over a barrier and then
+//   written over the primitives. FP64 16x12, 256 threads: 26.4 KB, six blocks per CU.
+// - the loads of the conserved states are issued before the wait for the CFL words.
+// - the tile follows the grid's size (ek_launch.h).
+// Per step, before -> now: FP64 64^2 9.4 -> 6.9 us, 512^2 17.4 -> 16.0, 2048^2 214 -> 188; FP32
+// 64^2 8.0 -> 5.9, 1000x333 (two-shock) 14.4 -> 13.6, 1024^2 29.5 -> 25.3.
 // ------------------------------------------------------------------------------------
-// One TX x TY tile of the 2D step, origin (i0, j0), with time step dt. Returns this
-// thread's contribution to the CFL maximum of the new state. Shared by the single-grid
-// kernel below and the batched (job pool) kernel.
-template <class T, int TX, int TY, int NT, int RS, int ST>
-__device__ __forceinline__ double hydro2d_tile(const T* __restrict__ Uin, T* __restrict__ Uout,
-                                               const Geom<T>& geo, const Gas<T>& gas, double dt, int i0, int j0)
+template <class T, int TX, int TY, int NT>
+struct Tile2 {
+  static constexpr int NV = 4;
+  static constexpr int QX = TX + 4, QY = TY + 4, QN = QX * QY;  // primitives: tile and 2-cell halo
+  static constexpr int PT = TX * TY, PH = 2 * TY + 2 * TX;      // traced cells: tile, halo cross
+  static constexpr int FXN = TX + 1, NFX = FXN * TY, NFY = TX * (TY + 1); // faces
+  static constexpr int OY = 2 * NV * NFX, NS = OY + 2 * NV * NFY;         // face states: x, then y
+  static constexpr int RQ = (QN + NT - 1) / NT;                           // loads per thread
+};
+
+// The conserved states of the tile and its 2-cell halo, ghosts resolved through the boundary map
+template <class T, int TX, int TY, int NT>
+struct Loaded2 {
+  using L = Tile2<T, TX, TY, NT>;
+  T u[L::RQ][4];
+  bool nx[L::RQ], ny[L::RQ];
+};
+
+template <class T, int TX, int TY, int NT>
+__device__ __forceinline__ void hydro2d_load(const T* __restrict__ Uin, const Geom<T>& geo, int i0, int j0,
+                                             Loaded2<T, TX, TY, NT>& in)
 {
-  constexpr int NV = 4;
-  constexpr int QX = TX + 4, QY = TY + 4, QN = QX * QY;
-  __shared__ T sQ[NV][QN];
-  __shared__ T sX[2][NV][TY][TX + 1]; // [0]: left state at face f (cell f-1), [1]: right state (cell f)
-  __shared__ T sY[2][NV][TY + 1][TX];
+  using L = Tile2<T, TX, TY, NT>;
+#pragma unroll
+  for (int r = 0; r < L::RQ; r++) {
+    const int w = (int)threadIdx.x + r * NT;
+    if (w < L::QN) {
+      const int si = bc_map(i0 - 2 + w % L::QX, geo.nx, geo.bc[0], geo.bc[1], in.nx[r]);
+      const int sj = bc_map(j0 - 2 + w / L::QX, geo.ny, geo.bc[2], geo.bc[3], in.ny[r]);
+      const long long o = (long long)sj * geo.nx + si;
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        in.u[r][v] = Uin[v * geo.vstride + o];
+    }
+  }
+}
+
+// One TX x TY tile of the 2D step, origin (i0, j0), with time step dt, from the states that
+// hydro2d_load fetched. Returns this thread's contribution to the CFL maximum of the new state.
+// Shared by the single-grid kernel below and the batched (job pool) kernel.
+template <class T, int TX, int TY, int NT, int RS, int ST, bool CMP>
+__device__ __forceinline__ double hydro2d_tile(const T* __restrict__ Uin, T* __restrict__ Uout,
+                                               const Geom<T>& geo, const Gas<T>& gas, double dt, int i0, int j0,
+                                               Loaded2<T, TX, TY, NT>& in)
+{
+  using L = Tile2<T, TX, TY, NT>;
+  constexpr int NV = L::NV, QX = L::QX, QN = L::QN, PT = L::PT, PH = L::PH, NFX = L::NFX, NFY = L::NFY;
+  static_assert(!CMP || NT >= PT + PH, "one traced cell per thread");
+  __shared__ T smem[CMP ? (L::NS > NV * QN ? L::NS : NV * QN) : L::NS + NV * QN];
+  T* const sQ = smem;
+  T* const sF = smem + (CMP ? 0 : NV * QN);
+  // state of side s (0: left, cell before the face; 1: right) at x face (fx, fy) / y face (fx, fy)
+  auto sX = [&](int s, int v, int fy, int fx) -> T& { return sF[(s * NV + v) * NFX + fy * L::FXN + fx]; };
+  auto sY = [&](int s, int v, int fy, int fx) -> T& { return sF[L::OY + (s * NV + v) * NFY + fy * TX + fx]; };
 
   const int tid = threadIdx.x;
   const T dtdx[2] = { T(dt / geo.dx), T(dt / geo.dy) };
   const int nx = geo.nx, ny = geo.ny;
 
-  // primitives of the tile plus a 2-cell halo, ghosts resolved through the boundary map
-  for (int w = tid; w < QN; w += NT) {
-    const int qx = w % QX, qy = w / QX;
-    bool nx_, ny_;
-    const int si = bc_map(i0 - 2 + qx, nx, geo.bc[0], geo.bc[1], nx_);
-    const int sj = bc_map(j0 - 2 + qy, ny, geo.bc[2], geo.bc[3], ny_);
-    const long long o = (long long)sj * nx + si;
-    T u[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++)
-      u[v] = Uin[v * geo.vstride + o];
-    if (nx_)
-      u[IU] = u[IU] * T(-1);
-    if (ny_)
-      u[IV] = u[IV] * T(-1);
-    T q[NV];
-    prims<T, 2>(gas, u, q);
+  for (int r = 0; r < L::RQ; r++) {
+    const int w = tid + r * NT;
+    if (w < QN) {
+      T* u = in.u[r];
+      if (in.nx[r])
+        u[IU] = u[IU] * T(-1);
+      if (in.ny[r])
+        u[IV] = u[IV] * T(-1);
+      T q[NV];
+      prims<T, 2>(gas, u, q);
 #pragma unroll
-    for (int v = 0; v < NV; v++)
-      sQ[v][w] = q[v];
+      for (int v = 0; v < NV; v++)
+        sQ[v * QN + w] = q[v];
+    }
   }
   __syncthreads();
 
   // slopes + face states: tile cells give 4 states, halo cells the one state a tile face needs
-  constexpr int PT = TX * TY, PH = 2 * TY + 2 * TX;
-  for (int w = tid; w < PT + PH; w += NT) {
-    int cx, cy;
-    unsigned want;
+  T fm[3][5], fp[3][5];
+  int cx, cy;
+  unsigned want;
+  auto trace = [&](int w) {
     if (w < PT) {
       cx = w % TX;
       cy = w / TX;
@@ -418,71 +465,84 @@ __device__ __forceinline__ double hydro2d_tile(const T* __restrict__ Uin, T* __r
     T q[NV], dq[3][5];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      q[v] = sQ[v][c];
+      const T* s = sQ + v * QN;
+      q[v] = s[c];
       if constexpr (ST == 0) {
         dq[0][v] = T(0);
         dq[1][v] = T(0);
       } else {
-        dq[0][v] = slope1<T, ST>(q[v], sQ[v][c + 1], sQ[v][c - 1]);
-        dq[1][v] = slope1<T, ST>(q[v], sQ[v][c + QX], sQ[v][c - QX]);
+        dq[0][v] = slope1<T, ST>(q[v], s[c + 1], s[c - 1]);
+        dq[1][v] = slope1<T, ST>(q[v], s[c + QX], s[c - QX]);
       }
     }
-    T fm[3][5], fp[3][5];
     trace_cell<T, 2>(gas, q, dq, dtdx, want, fm, fp);
+  };
+  auto store = [&] {
     if (want & 0x2) {
 #pragma unroll
       for (int v = 0; v < NV; v++)
-        sX[0][v][cy][cx + 1] = fm[0][v];
+        sX(0, v, cy, cx + 1) = fm[0][v];
     }
     if (want & 0x1) {
 #pragma unroll
       for (int v = 0; v < NV; v++)
-        sX[1][v][cy][cx] = fp[0][v];
+        sX(1, v, cy, cx) = fp[0][v];
     }
     if (want & 0x8) {
 #pragma unroll
       for (int v = 0; v < NV; v++)
-        sY[0][v][cy + 1][cx] = fm[1][v];
+        sY(0, v, cy + 1, cx) = fm[1][v];
     }
     if (want & 0x4) {
 #pragma unroll
       for (int v = 0; v < NV; v++)
-        sY[1][v][cy][cx] = fp[1][v];
+        sY(1, v, cy, cx) = fp[1][v];
+    }
+  };
+  if constexpr (CMP) {
+    if (tid < PT + PH)
+      trace(tid);
+    __syncthreads(); // every read of the primitives is done
+    if (tid < PT + PH)
+      store();
+  } else {
+    for (int w = tid; w < PT + PH; w += NT) {
+      trace(w);
+      store();
     }
   }
   __syncthreads();
 
   // Riemann problems: x faces (no swap), y faces (IU<->IV swapped around the solve)
-  constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1);
   for (int w = tid; w < NFX + NFY; w += NT) {
     T ql[NV], qr[NV], f[NV];
     if (w < NFX) {
-      const int fx = w % (TX + 1), fy = w / (TX + 1);
+      const int fx = w % L::FXN, fy = w / L::FXN;
 #pragma unroll
       for (int v = 0; v < NV; v++) {
-        ql[v] = sX[0][v][fy][fx];
-        qr[v] = sX[1][v][fy][fx];
+        ql[v] = sX(0, v, fy, fx);
+        qr[v] = sX(1, v, fy, fx);
       }
       riemann<T, NV, RS>(gas, ql, qr, f);
 #pragma unroll
       for (int v = 0; v < NV; v++)
-        sX[0][v][fy][fx] = f[v] * dtdx[0];
+        sX(0, v, fy, fx) = f[v] * dtdx[0];
     } else {
       const int h = w - NFX;
       const int fx = h % TX, fy = h / TX;
 #pragma unroll
       for (int v = 0; v < NV; v++) {
-        ql[v] = sY[0][v][fy][fx];
-        qr[v] = sY[1][v][fy][fx];
+        ql[v] = sY(0, v, fy, fx);
+        qr[v] = sY(1, v, fy, fx);
       }
       T t;
       t = ql[IU]; ql[IU] = ql[IV]; ql[IV] = t;
       t = qr[IU]; qr[IU] = qr[IV]; qr[IV] = t;
       riemann<T, NV, RS>(gas, ql, qr, f);
-      sY[0][ID][fy][fx] = f[ID] * dtdx[1];
-      sY[0][IP][fy][fx] = f[IP] * dtdx[1];
-      sY[0][IU][fy][fx] = f[IV] * dtdx[1];
-      sY[0][IV][fy][fx] = f[IU] * dtdx[1];
+      sY(0, ID, fy, fx) = f[ID] * dtdx[1];
+      sY(0, IP, fy, fx) = f[IP] * dtdx[1];
+      sY(0, IU, fy, fx) = f[IV] * dtdx[1];
+      sY(0, IV, fy, fx) = f[IU] * dtdx[1];
     }
   }
   __syncthreads();
@@ -490,18 +550,18 @@ __device__ __forceinline__ double hydro2d_tile(const T* __restrict__ Uin, T* __r
   // update (UpdateFunctor2D order: +Fx(i) -Fx(i+1) +Fy(j) -Fy(j+1)) and CFL of the new state
   double local = 0.0;
   for (int w = tid; w < PT; w += NT) {
-    const int cx = w % TX, cy = w / TX;
-    const int gi = i0 + cx, gj = j0 + cy;
+    const int x = w % TX, y = w / TX;
+    const int gi = i0 + x, gj = j0 + y;
     if (gi < nx && gj < ny) {
       const long long o = (long long)gj * nx + gi;
       T u[NV];
 #pragma unroll
       for (int v = 0; v < NV; v++) {
         T a = Uin[v * geo.vstride + o];
-        a += sX[0][v][cy][cx];
-        a -= sX[0][v][cy][cx + 1];
-        a += sY[0][v][cy][cx];
-        a -= sY[0][v][cy + 1][cx];
+        a += sX(0, v, y, x);
+        a -= sX(0, v, y, x + 1);
+        a += sY(0, v, y, x);
+        a -= sY(0, v, y + 1, x);
         u[v] = a;
         Uout[v * geo.vstride + o] = a;
       }
@@ -512,7 +572,7 @@ __device__ __forceinline__ double hydro2d_tile(const T* __restrict__ Uin, T* __r
   return local;
 }
 
-template <class T, int TX, int TY, int NT, int RS, int ST>
+template <class T, int TX, int TY, int NT, int RS, int ST, bool CMP>
 __global__ __launch_bounds__(NT) void hydro2d_step(const T* __restrict__ Uin, T* __restrict__ Uout,
                                                    Geom<T> geo, Gas<T> gas, StepCtl ctl)
 {
@@ -520,16 +580,35 @@ __global__ __launch_bounds__(NT) void hydro2d_step(const T* __restrict__ Uin, T*
   const bool first_block = blockIdx.x == 0;
   const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(geo.nx + TX - 1) / TX;
   const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
+  Loaded2<T, TX, TY, NT> in;
+  hydro2d_load<T, TX, TY, NT>(Uin, geo, i0, j0, in);
   double dt;
   TimeSlot cur;
   if (!step_begin(ctl, first_block, dt, cur))
     return;
-  const double local =
-      hydro2d_tile<T, TX, TY, NT, RS, ST>(Uin, Uout, geo, gas, dt, i0, j0);
+  const double local = hydro2d_tile<T, TX, TY, NT, RS, ST, CMP>(Uin, Uout, geo, gas, dt, i0, j0, in);
   block_max_to<NT>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x), local, sred);
   if (first_block && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);
 }
+
+// Tiles of a launch with many blocks and of one with few. FP64 (us per step at 512^2, 1024^2,
+// 2048^2): 16x12 16.0, 46, 188; 12x16 16.2, 47, 187; 14x14 17.1, -, 195; 24x8 16.3, 47, 188; 12x12
+// with 192 threads 17.0, 51, 197; 16x8 with 192 16.4, -, 209; 30x14 with 512 17.6, -, 193. FP32 has
+// the LDS for both arrays side by side and less to gain from more blocks: a larger tile repeats
+// less halo work (1024^2, 1400x1100: 32x16 25.3, 36.6; 64x8 26.0, 36.3; 32x12 CMP 26.0, 35.9;
+// 16x12 CMP 29.7, 44.0; 16x16 28.9, 43.5; 32x16 CMP with 640 threads 31.7, 44.6).
+template <class T>
+struct Tile2Of {
+  static constexpr bool F64 = sizeof(T) == 8;
+  static constexpr int X = F64 ? 16 : 32, Y = F64 ? 12 : 16, NT = F64 ? 256 : 512;
+  static constexpr bool CMP = F64;
+};
+// one pass per phase: 240 primitives, 176 traced cells, 280 faces for 320 threads
+struct SmallTile2 {
+  static constexpr int X = 16, Y = 8, NT = 320;
+  static constexpr bool CMP = true;
+};
 
 // ------------------------------------------------------------------------------------
 // CFL reduction over the current state (ComputeDtFunctor2D/3D), into slot `slot`.

@@ -8,24 +8,53 @@
 
 namespace ek {
 
-// Tile shapes. 2D: 16x16 cells per block (256 threads). 3D: T3X x T3Y column tiles marching
-// over z-chunks (ek_hydro3d.h; N3T threads: one per primitive column of the tile and its
-// 2-cell halo).
-constexpr int T2X = 16, T2Y = 16, N2T = 256;
+// 3D tiles: T3X x T3Y columns marching over z-chunks (ek_hydro3d.h; N3T threads: one per
+// primitive column of the tile and its 2-cell halo).
+//
+// 2D tiles (Tile2Of, ek_hydro.h). A grid that leaves CUs idle takes small ones with so many
+// threads that every phase is one pass; a step of it then lasts as long as its fullest CU, so
+// the line lies where the small tiles put no more blocks on one CU than the large ones do
+// (FP64, us per step, small / large tiles: 128^2 6.9 / 7.3, 200^2 8.2 / 7.4, 256^2 8.3 / 8.8,
+// 280^2 9.5 / 8.8, 512^2 19.6 / 16.0). In FP32 a second block on a CU costs the small tiles little
+// (64^2 5.9 / 7.8, 200^2 6.4 / 7.8, 256^2 6.5 / 7.9, 320^2 8.1 / 7.9, 512^2 12.7 / 9.8).
+template <class T>
+inline bool small_tile2(int nx, int ny)
+{
+  constexpr long long CUS = 256;
+  using S = SmallTile2;
+  using L = Tile2Of<T>;
+  const long long ns = (long long)((nx + S::X - 1) / S::X) * ((ny + S::Y - 1) / S::Y);
+  const long long nl = (long long)((nx + L::X - 1) / L::X) * ((ny + L::Y - 1) / L::Y);
+  return ns <= CUS || (ns <= 2 * CUS && (sizeof(T) == 4 || nl > CUS));
+}
 
 template <class T>
 using Step2Fn = void (*)(const T*, T*, Geom<T>, Gas<T>, StepCtl);
 template <class T>
 using Step3Fn = void (*)(const T*, T*, Geom<T>, Gas<T>, StepCtl, int, int, int, int);
 
-template <class T, int RS>
+template <class T, class C, int RS>
 inline Step2Fn<T> pick2(int st)
 {
   if (st == 0)
-    return hydro2d_step<T, T2X, T2Y, N2T, RS, 0>;
+    return hydro2d_step<T, C::X, C::Y, C::NT, RS, 0, C::CMP>;
   if (st == 1)
-    return hydro2d_step<T, T2X, T2Y, N2T, RS, 1>;
-  return hydro2d_step<T, T2X, T2Y, N2T, RS, 2>;
+    return hydro2d_step<T, C::X, C::Y, C::NT, RS, 1, C::CMP>;
+  return hydro2d_step<T, C::X, C::Y, C::NT, RS, 2, C::CMP>;
+}
+template <class T, class C>
+inline void launch2(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, const Gas<T>& gas, const StepCtl& ctl,
+                    hipStream_t s)
+{
+  Step2Fn<T> f;
+  switch (rs) {
+    case RS_APPROX: f = pick2<T, C, RS_APPROX>(st); break;
+    case RS_LLF: f = pick2<T, C, RS_LLF>(st); break;
+    case RS_HLL: f = pick2<T, C, RS_HLL>(st); break;
+    default: f = pick2<T, C, RS_HLLC>(st); break;
+  }
+  dim3 grid((unsigned)((geo.nx + C::X - 1) / C::X) * (unsigned)((geo.ny + C::Y - 1) / C::Y));
+  hipLaunchKernelGGL(f, grid, dim3(C::NT), 0, s, Uin, Uout, geo, gas, ctl);
 }
 template <class T, int RS>
 inline Step3Fn<T> pick3(int st)
@@ -42,15 +71,10 @@ inline hipError_t launch_step(int dim, int rs, int st, const T* Uin, T* Uout, co
                               const Gas<T>& gas, const StepCtl& ctl, int cz, hipStream_t s)
 {
   if (dim == 2) {
-    Step2Fn<T> f;
-    switch (rs) {
-      case RS_APPROX: f = pick2<T, RS_APPROX>(st); break;
-      case RS_LLF: f = pick2<T, RS_LLF>(st); break;
-      case RS_HLL: f = pick2<T, RS_HLL>(st); break;
-      default: f = pick2<T, RS_HLLC>(st); break;
-    }
-    dim3 grid((unsigned)((geo.nx + T2X - 1) / T2X) * (unsigned)((geo.ny + T2Y - 1) / T2Y));
-    hipLaunchKernelGGL(f, grid, dim3(N2T), 0, s, Uin, Uout, geo, gas, ctl);
+    if (small_tile2<T>(geo.nx, geo.ny))
+      launch2<T, SmallTile2>(rs, st, Uin, Uout, geo, gas, ctl, s);
+    else
+      launch2<T, Tile2Of<T>>(rs, st, Uin, Uout, geo, gas, ctl, s);
   } else {
     Step3Fn<T> f;
     switch (rs) {

@@ -240,8 +240,10 @@ static int upload_record(ek_pool* p, int id)
 static void tiles_of(const ek_pool* p, const ek_params& j, int& ntx, int& nty, int& ntz)
 {
   if (j.dim == 2) {
-    ntx = (j.nx + ek::pool::V2[p->variant][0] - 1) / ek::pool::V2[p->variant][0];
-    nty = (j.ny + ek::pool::V2[p->variant][1] - 1) / ek::pool::V2[p->variant][1];
+    const ek::pool::PoolTile2 t =
+        p->fp64 ? ek::pool::pool_tile2<double>(p->variant) : ek::pool::pool_tile2<float>(p->variant);
+    ntx = (j.nx + t.x - 1) / t.x;
+    nty = (j.ny + t.y - 1) / t.y;
     ntz = 1;
   } else {
     ntx = (j.nx + ek::pool::P3X - 1) / ek::pool::P3X;
@@ -518,7 +520,7 @@ extern "C" int ek_pool_create(const ek_params* kind, long long arena_bytes, int 
   p->jobs.resize(max_jobs);
   p->jev.assign(max_jobs, nullptr);
   p->freel[0] = p->cap;
-  p->variant = (kind->dim == 2 || mhd3) ? 0 : 2; // 16x16 tiles (2D), 32-plane chunks (3D) until tuned
+  p->variant = (kind->dim == 2 || mhd3) ? 0 : 2; // the first tile (2D), 32-plane chunks (3D) until tuned
   int dev = 0;
   hipError_t e;
   const size_t recb = record_bytes(p);

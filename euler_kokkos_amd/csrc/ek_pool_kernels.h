@@ -46,7 +46,7 @@ struct PoolWork {
   int tz_first; // z chunk * 2 + (1 if this item does the job's bookkeeping)
 };
 
-template <class T, int TX, int TY, int NT, int RS, int ST>
+template <class T, int TX, int TY, int NT, int RS, int ST, bool CMP>
 __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
                                                         const PoolWork* __restrict__ work,
@@ -66,12 +66,14 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
   ctl.tEnd = J.tEnd;
   ctl.nStepmax = J.nStepmax;
   const bool first = (it.tz_first & 1) != 0;
+  Loaded2<T, TX, TY, NT> in;
+  hydro2d_load<T, TX, TY, NT>(Ua + J.off, J.geo, it.tx * TX, it.ty * TY, in);
   double dt;
   TimeSlot cur;
   if (!step_begin(ctl, first, dt, cur))
     return;
   const double local =
-      hydro2d_tile<T, TX, TY, NT, RS, ST>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt, it.tx * TX, it.ty * TY);
+      hydro2d_tile<T, TX, TY, NT, RS, ST, CMP>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt, it.tx * TX, it.ty * TY, in);
   block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
   if (first && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);

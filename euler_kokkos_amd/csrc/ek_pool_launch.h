@@ -7,9 +7,28 @@
 namespace ek {
 namespace pool {
 
-// 2D tile shapes the autotuner chooses from: (TX, TY, threads)
+// 2D tiles the autotuner chooses from (Tile2Of, SmallTile2: ek_hydro.h); the first until tuned.
+// us per step of 24 ragged jobs of up to 320^2, then 100 of up to 512^2 in FP64 / 256 in FP32:
+// FP64 16x12 52.6, 422; 24x8 51.0, 425; small 65.9, 596 (16x16 with 47.6 KB of LDS 58.5, 486).
+// FP32 32x8 29.2, 616; 32x16 29.8, 569; 16x16 28.8, 663; small 41.2, 1010 (16x16 with the loads
+// after the CFL words 29.6, 809). 8 jobs of up to 64^2: small 6.8 and 5.8, the others 7.4 to 7.6.
+struct PoolTile2 {
+  int x, y, nt;
+  bool cmp;
+};
 constexpr int N2VARIANTS = 4;
-constexpr int V2[N2VARIANTS][3] = { { 16, 16, 256 }, { 32, 8, 256 }, { 16, 8, 128 }, { 8, 8, 64 } };
+template <class T>
+constexpr PoolTile2 pool_tile2(int v)
+{
+  using L = Tile2Of<T>;
+  using S = SmallTile2;
+  switch (v) {
+    case 0: return sizeof(T) == 8 ? PoolTile2{ L::X, L::Y, L::NT, L::CMP } : PoolTile2{ 32, 8, 256, false };
+    case 1: return { S::X, S::Y, S::NT, S::CMP };
+    case 2: return sizeof(T) == 8 ? PoolTile2{ 24, 8, 256, true } : PoolTile2{ L::X, L::Y, L::NT, L::CMP };
+    default: return sizeof(T) == 8 ? PoolTile2{ 12, 16, 256, true } : PoolTile2{ 16, 16, 256, false };
+  }
+}
 // 3D column tile (the z chunk depth is the tuned parameter)
 constexpr int P3X = 16, P3Y = 8, P3T = 256;
 
@@ -19,7 +38,8 @@ using Pool2Fn = void (*)(const T*, T*, const PoolJob<T>*, const PoolWork*, TimeS
 template <class T, int V, int ST>
 inline Pool2Fn<T> pick2v()
 {
-  return hydro2d_pool_step<T, V2[V][0], V2[V][1], V2[V][2], RS_HLLC, ST>;
+  constexpr PoolTile2 t = pool_tile2<T>(V);
+  return hydro2d_pool_step<T, t.x, t.y, t.nt, RS_HLLC, ST, t.cmp>;
 }
 
 template <class T>
@@ -52,7 +72,7 @@ inline hipError_t launch_step(int dim, int variant, int st, const T* Ua, T* Ub, 
   if (nwork <= 0)
     return hipSuccess;
   if (dim == 2)
-    hipLaunchKernelGGL(pick2<T>(variant, st), dim3(nwork), dim3(V2[variant][2]), 0, s, Ua, Ub, jobs, work, ts,
+    hipLaunchKernelGGL(pick2<T>(variant, st), dim3(nwork), dim3(pool_tile2<T>(variant).nt), 0, s, Ua, Ub, jobs, work, ts,
                        slot);
   else
     hipLaunchKernelGGL(pick3<T>(st), dim3(nwork), dim3(P3T), 0, s, Ua, Ub, jobs, work, ts, slot);
