@@ -531,8 +531,7 @@ enum Rec {
 };
 
 // ------------------------------------------------------------------------------------
-// The step kernel. TX x TY cells per block of NT threads; (TX+2)*(TY+2) must equal NT
-// (one trace record per thread).
+// The step kernel. TX x TY cells per block of NT threads, at least one per trace record.
 // ------------------------------------------------------------------------------------
 template <int TX, int TY>
 struct Tile {
@@ -542,18 +541,13 @@ struct Tile {
   static constexpr int BYX = TX + 2, BYY = TY + 3, BYN = BYX * BYY; // y faces: cols -1..TX, -1..TY+1
   static constexpr int RX = TX + 2, RN = (TX + 2) * (TY + 2);        // trace cells -1..TX
   static constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1), NE = (TX + 1) * (TY + 1);
-  // shared memory regions (in reals)
-  static constexpr int R1 = (NV * QN > 6 * NFX + 6 * NFY + NE) ? NV * QN : 6 * NFX + 6 * NFY + NE;
-  static constexpr int R2 = (NREC * RN > EN) ? NREC * RN : EN;
-  static constexpr int R3 = 2 * QN + 2 * AXN + 2 * BYN;
-  static constexpr int TOTAL = R1 + R2 + R3;
-  // compact layout: region CX holds, in turn, the primitives + edge fields + raw face fields
-  // (phases A-B1), the trace records (C) and the fluxes and EMFs (D); region CY the half-step
-  // face fields and transverse slopes (B0-C). The records and the Riemann results are
+  // shared memory (in reals): region CX holds, in turn, the primitives + edge fields + raw face
+  // fields (phases A-B1), the trace records (C) and the fluxes and EMFs (D); region CY the
+  // half-step face fields and transverse slopes (B0-C). The records and the Riemann results are
   // produced in registers and written after a barrier, so no two of them share the LDS.
   static constexpr int XA = NV * QN + EN + 2 * QN, XB = NREC * RN, XC = 6 * NFX + 6 * NFY + NE;
   static constexpr int CX = XA > XB ? (XA > XC ? XA : XC) : (XB > XC ? XB : XC);
-  static constexpr int CTOTAL = CX + 2 * AXN + 2 * BYN;
+  static constexpr int TOTAL = CX + 2 * AXN + 2 * BYN;
 };
 
 template <class T>
@@ -563,78 +557,95 @@ __device__ __forceinline__ void floor_dp(const Gas<T>& g, T& r, T& p)
   p = emax(g.smallp * r, p);
 }
 
-// WPE: waves per SIMD the registers are sized for. CMP: the compact LDS layout of Tile
-// (two more barriers per step): the FP32 30x14 tile (512 threads) takes 53.7 KB with it,
-// three blocks per CU, against 82 KB and two without. FP64 14x14 (256 threads) keeps the
-// plain layout (81 KB, two blocks per CU): at three blocks the two extra barriers and the
-// held results cost more than the third wave gains.
-template <class T, int TX, int TY, int NT, int RS, int ST, bool CMP, int WPE>
+// Issue bounds a large grid (FP64 60 % VALU busy with 14x14 tiles and all regions side by side:
+// 81 KB, two blocks of four waves per CU), latency a small one (loads, seven barriers, chains of
+// divisions and roots). With one region reused FP64 27x11 takes 79 KB for eight waves and 110
+// registers: sixteen waves per CU. A phase's work comes in whole waves of 64 items, so the tiles
+// (ek_mhd_launch.h) are those whose phases need few rounds of a block's waves: 27x11 has 10 waves
+// of faces and 6 of edges for 8 waves, 14x10 five and three for 4, 14x6 three and two for 5.
+// Per step, before -> now: FP64 48^2 16.3 -> 11.5 us, 300x211 22.1 -> 18.5, 1024^2 197 -> 169;
+// FP32 48^2 14.7 -> 8.6, 300x211 14.8 -> 12.0, 1024^2 80 -> 80. WPE: waves per SIMD the registers
+// are sized for.
+template <class T, int TX, int TY, int NT, int RS, int ST, int WPE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) void mhd2d_step(const T* __restrict__ Uin, T* __restrict__ Uout, Geom<T> geo,
                                                  Gas<T> gas, StepCtl ctl)
 {
   using L = Tile<TX, TY>;
-  static_assert(L::RN == NT, "one trace record per thread");
+  static_assert(L::RN <= NT, "one trace record per thread");
+  constexpr int RN = L::RN;
   static_assert(ST == 1 || ST == 2, "MHD trace supports slope_type 1 and 2");
   constexpr int QX = L::QX, QN = L::QN;
-  __shared__ T smem[CMP ? L::CTOTAL : L::TOTAL];
+  __shared__ T smem[L::TOTAL];
   __shared__ double sred[NT / 64];
   T* const sQ = smem;                                             // [NV][QN] primitives
   T* const sF = smem;                                             // after the trace: fluxes and EMFs
-  T* const sEz = smem + (CMP ? NV * QN : L::R1);                  // [EN] edge fields u*B - v*A
-  T* const sRec = CMP ? smem : smem + L::R1;                      // after the face evolution: [NREC][RN]
-  T* const sBf = smem + (CMP ? NV * QN + L::EN : L::R1 + L::R2);  // [2][QN] raw face fields (IA, IB)
-  T* const sAev = CMP ? smem + L::CX : sBf + 2 * QN;              // [AXN] half-step x-face field
+  T* const sEz = smem + NV * QN;                                  // [EN] edge fields u*B - v*A
+  T* const sRec = smem;                                           // after the face evolution: [NREC][RN]
+  T* const sBf = smem + NV * QN + L::EN;                          // [2][QN] raw face fields (IA, IB)
+  T* const sAev = smem + L::CX;                                   // [AXN] half-step x-face field
   T* const sDAy = sAev + L::AXN;         // [AXN] transverse slope dA/dy at x faces (halved)
   T* const sBev = sDAy + L::AXN;         // [BYN] half-step y-face field
   T* const sDBx = sBev + L::BYN;         // [BYN] transverse slope dB/dx at y faces (halved)
 
   const int tid = threadIdx.x;
   const bool first_block = blockIdx.x == 0;
-  double dt;
-  TimeSlot cur;
-  if (!step_begin(ctl, first_block, dt, cur))
-    return;
-  const T dtdx = T(dt / geo.dx), dtdy = T(dt / geo.dy);
   const int nx = geo.nx, ny = geo.ny;
   const long long vs = geo.vstride;
   const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(nx + TX - 1) / TX;
   const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
 
   // A: primitives and raw face fields on cells -2..TX+1 (ghosts through the boundary map;
-  // a reflecting x pass negates IU and IA, a reflecting y pass IV and IB)
-  for (int w = tid; w < QN; w += NT) {
-    const int lx = w % QX - 2, ly = w / QX - 2;
-    bool fx, fy, fx1, fy1;
-    const int si = bc_map(i0 + lx, nx, geo.bc[0], geo.bc[1], fx);
-    const int sj = bc_map(j0 + ly, ny, geo.bc[2], geo.bc[3], fy);
-    const int si1 = bc_map(i0 + lx + 1, nx, geo.bc[0], geo.bc[1], fx1);
-    const int sj1 = bc_map(j0 + ly + 1, ny, geo.bc[2], geo.bc[3], fy1);
-    const long long o = (long long)sj * nx + si;
-    T u[NV];
+  // a reflecting x pass negates IU and IA, a reflecting y pass IV and IB). The loads are issued
+  // before the wait for the CFL words.
+  constexpr int RQ = (QN + NT - 1) / NT;
+  T u[RQ][NV], mx[RQ], my[RQ];
+  bool fx[RQ], fy[RQ], fx1[RQ], fy1[RQ];
 #pragma unroll
-    for (int v = 0; v < NV; v++)
-      u[v] = Uin[v * vs + o];
-    if (fx) {
-      u[IU] = u[IU] * T(-1);
-      u[IA] = u[IA] * T(-1);
-    }
-    if (fy) {
-      u[IV] = u[IV] * T(-1);
-      u[IB] = u[IB] * T(-1);
-    }
-    T mx = Uin[IA * vs + (long long)sj * nx + si1];
-    if (fx1)
-      mx = mx * T(-1);
-    T my = Uin[IB * vs + (long long)sj1 * nx + si];
-    if (fy1)
-      my = my * T(-1);
-    T q[NV];
-    constoprim<T>(gas, u, mx, my, T(0), q);
+  for (int r = 0; r < RQ; r++) {
+    const int w = tid + r * NT;
+    if (w < QN) {
+      const int lx = w % QX - 2, ly = w / QX - 2;
+      const int si = bc_map(i0 + lx, nx, geo.bc[0], geo.bc[1], fx[r]);
+      const int sj = bc_map(j0 + ly, ny, geo.bc[2], geo.bc[3], fy[r]);
+      const int si1 = bc_map(i0 + lx + 1, nx, geo.bc[0], geo.bc[1], fx1[r]);
+      const int sj1 = bc_map(j0 + ly + 1, ny, geo.bc[2], geo.bc[3], fy1[r]);
+      const long long o = (long long)sj * nx + si;
 #pragma unroll
-    for (int v = 0; v < NV; v++)
-      sQ[v * QN + w] = q[v];
-    sBf[w] = u[IA];
-    sBf[QN + w] = u[IB];
+      for (int v = 0; v < NV; v++)
+        u[r][v] = Uin[v * vs + o];
+      mx[r] = Uin[IA * vs + (long long)sj * nx + si1];
+      my[r] = Uin[IB * vs + (long long)sj1 * nx + si];
+    }
+  }
+  double dt;
+  TimeSlot cur;
+  if (!step_begin(ctl, first_block, dt, cur))
+    return;
+  const T dtdx = T(dt / geo.dx), dtdy = T(dt / geo.dy);
+#pragma unroll
+  for (int r = 0; r < RQ; r++) {
+    const int w = tid + r * NT;
+    if (w < QN) {
+      if (fx[r]) {
+        u[r][IU] = u[r][IU] * T(-1);
+        u[r][IA] = u[r][IA] * T(-1);
+      }
+      if (fy[r]) {
+        u[r][IV] = u[r][IV] * T(-1);
+        u[r][IB] = u[r][IB] * T(-1);
+      }
+      if (fx1[r])
+        mx[r] = mx[r] * T(-1);
+      if (fy1[r])
+        my[r] = my[r] * T(-1);
+      T q[NV];
+      constoprim<T>(gas, u[r], mx[r], my[r], T(0), q);
+#pragma unroll
+      for (int v = 0; v < NV; v++)
+        sQ[v * QN + w] = q[v];
+      sBf[w] = u[r][IA];
+      sBf[QN + w] = u[r][IB];
+    }
   }
   __syncthreads();
 
@@ -686,7 +697,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
   __syncthreads();
 
   // B: trace record of cell (tid%RX - 1, tid/RX - 1)
-  {
+  T rv[NREC];
+  if (tid < RN) {
     const int lx = tid % L::RX - 1, ly = tid / L::RX - 1;
     const int c = (ly + 2) * QX + (lx + 2);
     T q[NV], dx_[NV], dy_[NV];
@@ -726,7 +738,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
     const T sA0 = (u * dBy + B * duy - v * dAy - A * dvy) * dtdy;
     const T sB0 = (-u * dBx - B * dux + v * dAx + A * dvx) * dtdx;
     const T sC0 = (w * dAx + A * dwx - u * dCx - C * dux) * dtdx + (-v * dCy - C * dvy + w * dBy + B * dwy) * dtdy;
-    T rv[NREC];
     rv[R_R] = r + sr0;
     rv[R_U] = u + su0;
     rv[R_V] = v + sv0;
@@ -749,11 +760,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
     rv[R_DPY] = dpy;
     rv[R_DAY] = dAy;
     rv[R_DCY] = dCy;
-    if constexpr (CMP)
-      __syncthreads(); // every read of the primitives and raw face fields is done
+  }
+  __syncthreads(); // every read of the primitives and raw face fields is done
+  if (tid < RN) {
 #pragma unroll
     for (int k = 0; k < NREC; k++)
-      sRec[k * NT + tid] = rv[k];
+      sRec[k * RN + tid] = rv[k];
   }
   __syncthreads();
 
@@ -765,7 +777,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
     constexpr int NF = L::NFX + L::NFY;
     constexpr int TF = (NF + 63) / 64, TE = (L::NE + 63) / 64;
     const int wid = tid >> 6, lane = tid & 63;
-    auto rec = [&](int cell, int k) -> T { return sRec[k * NT + cell]; };
+    auto rec = [&](int cell, int k) -> T { return sRec[k * RN + cell]; };
     // flux of face k (x faces first) as its solve returns it: ID IP IU IV IW IC, where a y
     // face's IU is the y momentum flux (rotated solve)
     auto face = [&](int k, T* out) {
@@ -891,164 +903,36 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
       floor_dp(gas, LB.r, LB.p);
       return emf_z<T>(gas, RT, RB, LT, LB);
     };
-    if constexpr (!CMP) {
-      // the same solves written out in place (the FP64 step built from the lambdas above
-      // measured 1.2 % slower: same instructions, scheduled differently)
-      for (int task = wid; task < TF + TE; task += NT / 64) {
-        if (task < TF) {
-          const int k = task * 64 + lane;
-          if (k < NF) {
-            T ql[NV], qr[NV], f[NV];
-            if (k < L::NFX) {
-              const int fxl = k % (TX + 1), y = k / (TX + 1);
-              const int cl = (y + 1) * L::RX + fxl, cr = cl + 1; // cells (fxl-1, y), (fxl, y)
-              const T a = sAev[(y + 1) * L::AXX + fxl + 1];
-              ql[ID] = rec(cl, R_R) + rec(cl, R_DRX);
-              ql[IU] = rec(cl, R_U) + rec(cl, R_DUX);
-              ql[IV] = rec(cl, R_V) + rec(cl, R_DVX);
-              ql[IW] = rec(cl, R_W) + rec(cl, R_DWX);
-              ql[IP] = rec(cl, R_P) + rec(cl, R_DPX);
-              ql[IA] = a;
-              ql[IB] = rec(cl, R_B) + rec(cl, R_DBX);
-              ql[IC] = rec(cl, R_C) + rec(cl, R_DCX);
-              floor_dp(gas, ql[ID], ql[IP]);
-              qr[ID] = rec(cr, R_R) - rec(cr, R_DRX);
-              qr[IU] = rec(cr, R_U) - rec(cr, R_DUX);
-              qr[IV] = rec(cr, R_V) - rec(cr, R_DVX);
-              qr[IW] = rec(cr, R_W) - rec(cr, R_DWX);
-              qr[IP] = rec(cr, R_P) - rec(cr, R_DPX);
-              qr[IA] = a;
-              qr[IB] = rec(cr, R_B) - rec(cr, R_DBX);
-              qr[IC] = rec(cr, R_C) - rec(cr, R_DCX);
-              floor_dp(gas, qr[ID], qr[IP]);
-            } else {
-              const int h = k - L::NFX;
-              const int x = h % TX, fyl = h / TX;
-              const int cb = fyl * L::RX + x + 1, ct = cb + L::RX; // cells (x, fyl-1), (x, fyl)
-              const T b = sBev[(fyl + 1) * L::BYX + x + 1];
-              // qm_y of the lower cell and qp_y of the upper one, then IU<->IV, IA<->IB
-              T r_ = rec(cb, R_R) + rec(cb, R_DRY);
-              T p_ = rec(cb, R_P) + rec(cb, R_DPY);
-              floor_dp(gas, r_, p_);
-              ql[ID] = r_;
-              ql[IP] = p_;
-              ql[IV] = rec(cb, R_U) + rec(cb, R_DUY);
-              ql[IU] = rec(cb, R_V) + rec(cb, R_DVY);
-              ql[IW] = rec(cb, R_W) + rec(cb, R_DWY);
-              ql[IB] = rec(cb, R_A) + rec(cb, R_DAY);
-              ql[IA] = b;
-              ql[IC] = rec(cb, R_C) + rec(cb, R_DCY);
-              r_ = rec(ct, R_R) - rec(ct, R_DRY);
-              p_ = rec(ct, R_P) - rec(ct, R_DPY);
-              floor_dp(gas, r_, p_);
-              qr[ID] = r_;
-              qr[IP] = p_;
-              qr[IV] = rec(ct, R_U) - rec(ct, R_DUY);
-              qr[IU] = rec(ct, R_V) - rec(ct, R_DVY);
-              qr[IW] = rec(ct, R_W) - rec(ct, R_DWY);
-              qr[IB] = rec(ct, R_A) - rec(ct, R_DAY);
-              qr[IA] = b;
-              qr[IC] = rec(ct, R_C) - rec(ct, R_DCY);
-            }
-            riemann<T, RS>(gas, ql, qr, f);
-            if (k < L::NFX) {
-              sFx[0 * L::NFX + k] = f[ID];
-              sFx[1 * L::NFX + k] = f[IP];
-              sFx[2 * L::NFX + k] = f[IU];
-              sFx[3 * L::NFX + k] = f[IV];
-              sFx[4 * L::NFX + k] = f[IW];
-              sFx[5 * L::NFX + k] = f[IC];
-            } else {
-              const int h = k - L::NFX;
-              sFy[0 * L::NFY + h] = f[ID];
-              sFy[1 * L::NFY + h] = f[IP];
-              sFy[2 * L::NFY + h] = f[IV];
-              sFy[3 * L::NFY + h] = f[IU];
-              sFy[4 * L::NFY + h] = f[IW];
-              sFy[5 * L::NFY + h] = f[IC];
-            }
-          }
-        } else {
-          const int k = (task - TF) * 64 + lane;
-          if (k < L::NE) {
-            const int cx = k % (TX + 1), cy = k / (TX + 1);
-            const int cLB = (cy + 1) * L::RX + cx + 1; // cell (cx, cy)
-            const int cRB = cLB - 1;                   // (cx-1, cy)
-            const int cLT = cLB - L::RX;               // (cx, cy-1)
-            const int cRT = cLT - 1;                   // (cx-1, cy-1)
-            const int aT = cy * L::AXX + cx + 1;       // x face cx, row cy-1
-            const int aB = aT + L::AXX;                // x face cx, row cy
-            const int bL = (cy + 1) * L::BYX + cx;     // y face cy, column cx-1
-            const int bR = bL + 1;                     // y face cy, column cx
-            Edge<T> RT, RB, LT, LB;
-            RT.r = rec(cRT, R_R) + (rec(cRT, R_DRX) + rec(cRT, R_DRY));
-            RT.u = rec(cRT, R_U) + (rec(cRT, R_DUX) + rec(cRT, R_DUY));
-            RT.v = rec(cRT, R_V) + (rec(cRT, R_DVX) + rec(cRT, R_DVY));
-            RT.p = rec(cRT, R_P) + (rec(cRT, R_DPX) + rec(cRT, R_DPY));
-            RT.a = sAev[aT] + sDAy[aT];
-            RT.b = sBev[bL] + sDBx[bL];
-            RT.c = rec(cRT, R_C) + (rec(cRT, R_DCX) + rec(cRT, R_DCY));
-            floor_dp(gas, RT.r, RT.p);
-            RB.r = rec(cRB, R_R) + (rec(cRB, R_DRX) - rec(cRB, R_DRY));
-            RB.u = rec(cRB, R_U) + (rec(cRB, R_DUX) - rec(cRB, R_DUY));
-            RB.v = rec(cRB, R_V) + (rec(cRB, R_DVX) - rec(cRB, R_DVY));
-            RB.p = rec(cRB, R_P) + (rec(cRB, R_DPX) - rec(cRB, R_DPY));
-            RB.a = sAev[aB] + (-sDAy[aB]);
-            RB.b = sBev[bL] + sDBx[bL];
-            RB.c = rec(cRB, R_C) + (rec(cRB, R_DCX) - rec(cRB, R_DCY));
-            floor_dp(gas, RB.r, RB.p);
-            LT.r = rec(cLT, R_R) + (-rec(cLT, R_DRX) + rec(cLT, R_DRY));
-            LT.u = rec(cLT, R_U) + (-rec(cLT, R_DUX) + rec(cLT, R_DUY));
-            LT.v = rec(cLT, R_V) + (-rec(cLT, R_DVX) + rec(cLT, R_DVY));
-            LT.p = rec(cLT, R_P) + (-rec(cLT, R_DPX) + rec(cLT, R_DPY));
-            LT.a = sAev[aT] + sDAy[aT];
-            LT.b = sBev[bR] + (-sDBx[bR]);
-            LT.c = rec(cLT, R_C) + (-rec(cLT, R_DCX) + rec(cLT, R_DCY));
-            floor_dp(gas, LT.r, LT.p);
-            LB.r = rec(cLB, R_R) + (-rec(cLB, R_DRX) - rec(cLB, R_DRY));
-            LB.u = rec(cLB, R_U) + (-rec(cLB, R_DUX) - rec(cLB, R_DUY));
-            LB.v = rec(cLB, R_V) + (-rec(cLB, R_DVX) - rec(cLB, R_DVY));
-            LB.p = rec(cLB, R_P) + (-rec(cLB, R_DPX) - rec(cLB, R_DPY));
-            LB.a = sAev[aB] + (-sDAy[aB]);
-            LB.b = sBev[bR] + (-sDBx[bR]);
-            LB.c = rec(cLB, R_C) + (-rec(cLB, R_DCX) - rec(cLB, R_DCY));
-            floor_dp(gas, LB.r, LB.p);
-            sE[k] = emf_z<T>(gas, RT, RB, LT, LB);
-          }
-        }
-      }
-    } else {
-      // the fluxes and EMFs go where the records are: every result is held until all
-      // records have been read (EMF tasks first, so that at most the EMF and one face's
-      // fluxes are held through a solve)
-      constexpr int NW = NT / 64, MAXT = (TF + TE + NW - 1) / NW;
-      T hold[MAXT][6];
+    // the fluxes and EMFs go where the records are: every result is held until all
+    // records have been read (EMF tasks first, so that at most the EMF and one face's
+    // fluxes are held through a solve)
+    constexpr int NW = NT / 64, MAXT = (TF + TE + NW - 1) / NW;
+    T hold[MAXT][6];
 #pragma unroll
-      for (int j = 0; j < MAXT; j++) {
-        const int task = wid + j * NW;
-        if (task < TE) {
-          const int k = task * 64 + lane;
-          if (k < L::NE)
-            hold[j][0] = edge(k);
-        } else if (task < TE + TF) {
-          const int k = (task - TE) * 64 + lane;
-          if (k < NF)
-            face(k, hold[j]);
-        }
+    for (int j = 0; j < MAXT; j++) {
+      const int task = wid + j * NW;
+      if (task < TE) {
+        const int k = task * 64 + lane;
+        if (k < L::NE)
+          hold[j][0] = edge(k);
+      } else if (task < TE + TF) {
+        const int k = (task - TE) * 64 + lane;
+        if (k < NF)
+          face(k, hold[j]);
       }
-      __syncthreads();
+    }
+    __syncthreads();
 #pragma unroll
-      for (int j = 0; j < MAXT; j++) {
-        const int task = wid + j * NW;
-        if (task < TE) {
-          const int k = task * 64 + lane;
-          if (k < L::NE)
-            sE[k] = hold[j][0];
-        } else if (task < TE + TF) {
-          const int k = (task - TE) * 64 + lane;
-          if (k < NF)
-            store_face(k, hold[j]);
-        }
+    for (int j = 0; j < MAXT; j++) {
+      const int task = wid + j * NW;
+      if (task < TE) {
+        const int k = task * 64 + lane;
+        if (k < L::NE)
+          sE[k] = hold[j][0];
+      } else if (task < TE + TF) {
+        const int k = (task - TE) * 64 + lane;
+        if (k < NF)
+          store_face(k, hold[j]);
       }
     }
   }

@@ -7,45 +7,80 @@
 namespace ek {
 namespace mhd {
 
-// Tile of the 2D MHD step: the (TX+2) x (TY+2) trace region gives one record per thread.
-// FP64: 14x14 cells, 256 threads (81 KB of LDS, two blocks per CU). FP32: 30x14, 512
-// threads, compact LDS layout (53.7 KB, three blocks per CU, 71 VGPRs, six waves per SIMD).
-// Per 1024^2 Orszag-Tang step: FP32 0.139 ms at 14x14, 0.097 at 30x14, 0.088 with the
-// compact layout; FP64 0.246 ms at 14x14, 0.260 at 30x14, 0.249 with the compact layout at
-// three waves per SIMD (every variant bitwise the same).
+// Tiles of the 2D MHD step. A launch lasts as long as the CU with the most blocks: about
+// A + B * ceil(blocks / 256) us, A and B measured on grids of 48^2 to 1024^2 (Orszag-Tang, HLLD)
+// for each tile; the launch takes the tile with the smallest. us per step, FP64 14x6 / 14x10 /
+// 27x11: 140^2 11.7 / 13.5 / 18.2, 200^2 16.0 / 18.1 / 18.2, 300^2 35 / 23.1 / 28.2, 700^2 155 /
+// 83.4 / 84.8, 1024^2 328 / 179 / 169 (14x14 in 81 KB: 16.6, 16.7, 22.5, 93.4, 197; 30x10 174,
+// 20x15 179 at 1024^2). FP32 14x6 / 14x10 / 30x14: 140^2 8.7 / 10.3 / 14.8, 240^2 11.5 / 11.9 /
+// 14.8, 300^2 14.9 / 14.1 / 15.0, 420^2 24.4 / 18.2 / 19.8, 700^2 56 / 38.6 / 37.8, 1024^2 115 /
+// 80.9 / 80.3 (27x11 86, 32x13 78 to 80).
 template <class T>
-struct M2Tile {
+struct M2Small {
   static constexpr bool F64 = sizeof(T) == 8;
-  static constexpr int X = F64 ? 14 : 30, Y = 14, NT = F64 ? 256 : 512;
-  static constexpr bool CMP = !F64;
-  static constexpr int WPE = F64 ? 2 : 6;
+  static constexpr int X = 14, Y = 6, NT = 320, WPE = F64 ? 4 : 8;
+  static constexpr double A = F64 ? 5.7 : 6.5, B = F64 ? 5.6 : 1.9;
+};
+template <class T>
+struct M2Mid {
+  static constexpr bool F64 = sizeof(T) == 8;
+  static constexpr int X = 14, Y = 10, NT = 256, WPE = F64 ? 4 : 8;
+  static constexpr double A = F64 ? 7.9 : 8.0, B = F64 ? 5.4 : 2.2;
+};
+template <class T>
+struct M2Large {
+  static constexpr bool F64 = sizeof(T) == 8;
+  static constexpr int X = F64 ? 27 : 30, Y = F64 ? 11 : 14, NT = 512, WPE = F64 ? 4 : 6;
+  static constexpr double A = F64 ? 7.0 : 8.7, B = F64 ? 11.3 : 5.8;
 };
 
 template <class T>
 using MStepFn = void (*)(const T*, T*, Geom<T>, Gas<T>, StepCtl);
 
-template <class T, int RS>
+template <class T, class M, int RS>
 inline MStepFn<T> pick(int st)
 {
-  using M = M2Tile<T>;
   if (st == 1)
-    return mhd2d_step<T, M::X, M::Y, M::NT, RS, 1, M::CMP, M::WPE>;
-  return mhd2d_step<T, M::X, M::Y, M::NT, RS, 2, M::CMP, M::WPE>;
+    return mhd2d_step<T, M::X, M::Y, M::NT, RS, 1, M::WPE>;
+  return mhd2d_step<T, M::X, M::Y, M::NT, RS, 2, M::WPE>;
+}
+
+template <class M, class T>
+inline long long blocks_of(const Geom<T>& geo)
+{
+  return (long long)((geo.nx + M::X - 1) / M::X) * ((geo.ny + M::Y - 1) / M::Y);
+}
+
+template <class M, class T>
+inline double estimate(const Geom<T>& geo)
+{
+  return M::A + M::B * (double)((blocks_of<M>(geo) + 255) / 256);
+}
+
+template <class T, class M>
+inline void launch_tiles(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, const Gas<T>& gas,
+                         const StepCtl& ctl, hipStream_t s)
+{
+  MStepFn<T> f;
+  switch (rs) {
+    case RS_HLL: f = pick<T, M, RS_HLL>(st); break;
+    case RS_LLF: f = pick<T, M, RS_LLF>(st); break;
+    default: f = pick<T, M, RS_HLLD>(st); break;
+  }
+  hipLaunchKernelGGL(f, dim3((unsigned)blocks_of<M>(geo)), dim3(M::NT), 0, s, Uin, Uout, geo, gas, ctl);
 }
 
 template <class T>
 inline hipError_t launch_step(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, const Gas<T>& gas,
                               const StepCtl& ctl, hipStream_t s)
 {
-  MStepFn<T> f;
-  switch (rs) {
-    case RS_HLL: f = pick<T, RS_HLL>(st); break;
-    case RS_LLF: f = pick<T, RS_LLF>(st); break;
-    default: f = pick<T, RS_HLLD>(st); break;
-  }
-  using M = M2Tile<T>;
-  dim3 grid((unsigned)((geo.nx + M::X - 1) / M::X) * (unsigned)((geo.ny + M::Y - 1) / M::Y));
-  hipLaunchKernelGGL(f, grid, dim3(M::NT), 0, s, Uin, Uout, geo, gas, ctl);
+  const double small = estimate<M2Small<T>>(geo), mid = estimate<M2Mid<T>>(geo);
+  if (estimate<M2Large<T>>(geo) < (small < mid ? small : mid))
+    launch_tiles<T, M2Large<T>>(rs, st, Uin, Uout, geo, gas, ctl, s);
+  else if (small < mid)
+    launch_tiles<T, M2Small<T>>(rs, st, Uin, Uout, geo, gas, ctl, s);
+  else
+    launch_tiles<T, M2Mid<T>>(rs, st, Uin, Uout, geo, gas, ctl, s);
   return hipGetLastError();
 }
 
