@@ -3,6 +3,7 @@
 #include "ek_hip.h"
 #include "ek_internal.h"
 #include "ek_geom_host.h"
+#include "ek_hostcopy.h"
 
 #include <algorithm>
 #include <cmath>
@@ -332,16 +333,7 @@ extern "C" int ek_download(ek_ctx* c, double* host, int layout)
   const int is = p.nx + 2 * p.gw, js = p.ny + 2 * p.gw, ks = p.nz + 2 * p.gw;
   if (layout == EK_LAYOUT_SOA) {
     const long long n = c->ncell * p.nbvar;
-    if (p.precision == EK_FP64) {
-      EK_HIP(c, hipMemcpyAsync(host, c->U[c->cur], n * 8, hipMemcpyDeviceToHost, c->stream));
-      EK_HIP(c, hipStreamSynchronize(c->stream));
-    } else {
-      std::vector<float> tmp(n);
-      EK_HIP(c, hipMemcpyAsync(tmp.data(), c->U[c->cur], n * 4, hipMemcpyDeviceToHost, c->stream));
-      EK_HIP(c, hipStreamSynchronize(c->stream));
-      for (long long i = 0; i < n; i++)
-        host[i] = (double)tmp[i];
-    }
+    EK_HIP(c, ek::copy_to_host(host, c->U[c->cur], p.precision != EK_FP64, n, c->stream));
   } else if (layout == EK_LAYOUT_REFERENCE) {
     const long long n = ref_elems(p);
     if (int r = ensure_stage(c, n))
@@ -352,8 +344,7 @@ extern "C" int ek_download(ek_ctx* c, double* host, int layout)
     else
       EK_HIP(c, ek::fp32::soa_to_ref(p.dim, (const float*)c->U[c->cur], c->stage, c->g32, p.gw, p.nbvar, is,
                                     js, ks, p.mhd, c->stream));
-    EK_HIP(c, hipMemcpyAsync(host, c->stage, n * 8, hipMemcpyDeviceToHost, c->stream));
-    EK_HIP(c, hipStreamSynchronize(c->stream));
+    EK_HIP(c, ek::copy_to_host(host, c->stage, false, n, c->stream));
   } else {
     return fail(c, EK_EINVAL, "unknown layout");
   }

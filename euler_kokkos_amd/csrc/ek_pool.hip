@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "ek_geom_host.h"
+#include "ek_hostcopy.h"
 #include "ek_internal.h"
 #include "ek_pool_launch.h"
 #include "ek_pool_mhd3d.h"
@@ -978,16 +979,7 @@ extern "C" int ek_pool_download(ek_pool* p, int id, double* host, int layout)
   const HostJob& h = p->jobs[id];
   const char* src = (const char*)p->A[job_parity(p, h)] + (size_t)h.off * p->elem;
   if (layout == EK_LAYOUT_SOA) {
-    if (p->fp64) {
-      PHIP(p, hipMemcpyAsync(host, src, (size_t)h.nelem * 8, hipMemcpyDeviceToHost, p->stream));
-      PHIP(p, hipStreamSynchronize(p->stream));
-    } else {
-      std::vector<float> tmp((size_t)h.nelem);
-      PHIP(p, hipMemcpyAsync(tmp.data(), src, (size_t)h.nelem * 4, hipMemcpyDeviceToHost, p->stream));
-      PHIP(p, hipStreamSynchronize(p->stream));
-      for (long long i = 0; i < h.nelem; i++)
-        host[i] = tmp[i];
-    }
+    PHIP(p, ek::copy_to_host(host, src, !p->fp64, h.nelem, p->stream));
     return EK_OK;
   }
   if (layout != EK_LAYOUT_REFERENCE)
@@ -1010,8 +1002,7 @@ extern "C" int ek_pool_download(ek_pool* p, int id, double* host, int layout)
     PHIP(p, ek::fp32::soa_to_ref(jp.dim, (const float*)src, p->stage, g, jp.gw, jp.nbvar, is, js, ks, jp.mhd,
                                  p->stream));
   }
-  PHIP(p, hipMemcpyAsync(host, p->stage, (size_t)nr * 8, hipMemcpyDeviceToHost, p->stream));
-  PHIP(p, hipStreamSynchronize(p->stream));
+  PHIP(p, ek::copy_to_host(host, p->stage, false, nr, p->stream));
   return EK_OK;
 }
 
