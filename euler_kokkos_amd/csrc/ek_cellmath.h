@@ -60,7 +60,7 @@ __device__ __forceinline__ bool signbit_of(float a) { return __float_as_int(a) <
 // (plain): fused into the sum it enters, FP32 results would differ from a division's.
 // With a division (and the library's root) everywhere, per step: 3D hydro 256^3 FP64 1.20 ms,
 // now 1.11, FP32 0.554 -> 0.531; 2D MHD 1024^2 FP64 0.250 -> 0.206, FP32 0.087 -> 0.078; 3D
-// MHD 128^3 FP64 1.34 -> 1.26 (same box, bitwise the same states; 3D MHD in FP32 is bound by
+// MHD 128^3 FP64 1.34 -> 1.26 (same GPU, bitwise the same states; 3D MHD in FP32 is bound by
 // bytes and stays).
 template <class T>
 struct Inv;

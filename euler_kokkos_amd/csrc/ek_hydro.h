@@ -212,9 +212,10 @@ __device__ __forceinline__ unsigned long long* reduce_word(unsigned long long* d
 
 // Position of block b of n in an order that gives each XCD a contiguous eighth of the grid
 // (blocks are dealt to the 8 XCDs round robin; the remainder keeps its place): neighbouring
-// tiles then share their halo lines in one XCD's L2 (per step, same box, in dispatch order ->
-// in this one: 2D hydro 64^2 9.6 -> 9.4 us, 512^2 19.8 -> 18.2, 1000x333 FP32 two-shock 18.5
-// -> 14.6; 2D MHD 300x211 26.0 -> 22.8, 1024^2 210 -> 206, FP32 84.1 -> 81.9).
+// tiles then share their halo lines in one XCD's L2 (per step, same GPU, in dispatch order ->
+// in this one, with 16x16 hydro and 14x14 or 30x14 MHD tiles: 2D hydro 64^2 9.6 -> 9.4 us,
+// 512^2 19.8 -> 18.2, 1000x333 FP32 two-shock 18.5 -> 14.6; 2D MHD 300x211 26.0 -> 22.8, 1024^2
+// 210 -> 206, FP32 84.1 -> 81.9).
 __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
 {
   const unsigned n8 = n / 8;
@@ -226,8 +227,8 @@ __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
 // round of blocks. With m blocks on `slots` places a launch takes about (chunk + a) *
 // (floor(m / slots) + b + (1 - b) frac) plane times, frac the part of the places an incomplete
 // last round fills (a block alone on its CU is faster per plane than one of several). Returns
-// the chunk length between lo and hi with the smallest estimate.
-inline int z_chunk_of(long long tiles, int n, int slots, double a, double b, int lo, int hi)
+// the chunk length between lo and hi with the smallest estimate, and that estimate in *time.
+inline int z_chunk_of(long long tiles, int n, int slots, double a, double b, int lo, int hi, double* time = nullptr)
 {
   int best = n < hi ? n : hi;
   double least = 1e300;
@@ -244,6 +245,8 @@ inline int z_chunk_of(long long tiles, int n, int slots, double a, double b, int
       best = cz;
     }
   }
+  if (time)
+    *time = least;
   return best;
 }
 
@@ -319,8 +322,8 @@ __device__ __forceinline__ void step_end_bookkeeping(const StepCtl& c, const Tim
 
 // CFL term of one cell of the new state. The FP64 state uses the reference's expression
 // as is; an FP32 state is widened so that the dt reduction always runs in FP64, with one
-// FP64 division (1/rho) where the reference's expression has five (FP32 3D step 0.553 ->
-// 0.538 ms at 256^3; the divisions by the cell size stay: a hoisted 1/dx costs registers).
+// FP64 reciprocal (1/rho) where the reference's expression has five divisions, and products
+// with 1/dx, 1/dy, 1/dz from the host.
 template <class T, int DIM>
 __device__ __forceinline__ double cfl_term(const Gas<T>& gas, const T* u, const Geom<T>& geo)
 {

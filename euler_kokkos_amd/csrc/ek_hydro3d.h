@@ -31,7 +31,7 @@
 
 namespace ek {
 
-// Column tile of the single-grid 3D step: 16 x 8 cells, 256 threads.
+// Column tile of the single-grid 3D step: 16 x 8 cells, 256 threads, or 8 x 16 ("turned").
 constexpr int T3X = 16, T3Y = 8, N3T = 256;
 
 // Blocks of the 3D step that 256 CUs hold at once: three per CU in FP64 (53.5 KB of LDS, 168
@@ -45,11 +45,19 @@ constexpr int T3SLOTS = 256 * (sizeof(T) == 8 ? 3 : 5);
 // (The longest chunk that gives 2048 blocks, the rule before it, is 13 % off on average:
 // 101x75x130 FP64 116 -> 95 us per step, FP32 54 -> 49; 128^3 174 -> 159 and 80 -> 73; 32^3 24.7
 // -> 17.7; 256^3 unchanged.)
+// Turned tiles have shorter rows to load (1 to 2 % slower at 64^3 and 256^3, FP32 up to 4 %) but
+// fill some grids with fewer tiles: they are taken where their estimate is 5 % lower (us per step,
+// 16x8 -> 8x16: 101x75x130 FP64 93.6 -> 89.7, FP32 47.2 -> 45.0; 24x180x90 49.1 -> 44.4 and 28.1 ->
+// 24.8), which the chunk length says with its sign: negative for turned tiles.
 template <class T>
 inline int hydro3d_z_chunk(int nx, int ny, int nz)
 {
-  const long long tiles = (long long)((nx + T3X - 1) / T3X) * ((ny + T3Y - 1) / T3Y);
-  return z_chunk_of(tiles, nz, T3SLOTS<T>, sizeof(T) == 8 ? 1.5 : 2.0, sizeof(T) == 8 ? 0.3 : 0.45, 2, 64);
+  const double a = sizeof(T) == 8 ? 1.5 : 2.0, b = sizeof(T) == 8 ? 0.3 : 0.45;
+  auto tiles = [&](int tx, int ty) { return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty); };
+  double t, turned;
+  const int cz = z_chunk_of(tiles(T3X, T3Y), nz, T3SLOTS<T>, a, b, 2, 64, &t);
+  const int czt = z_chunk_of(tiles(T3Y, T3X), nz, T3SLOTS<T>, a, b, 2, 64, &turned);
+  return turned < 0.95 * t ? -czt : cz;
 }
 
 template <int TX, int TY, int NT>

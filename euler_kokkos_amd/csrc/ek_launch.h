@@ -56,14 +56,27 @@ inline void launch2(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, c
   dim3 grid((unsigned)((geo.nx + C::X - 1) / C::X) * (unsigned)((geo.ny + C::Y - 1) / C::Y));
   hipLaunchKernelGGL(f, grid, dim3(C::NT), 0, s, Uin, Uout, geo, gas, ctl);
 }
-template <class T, int RS>
+template <class T, int TX, int TY, int RS>
 inline Step3Fn<T> pick3(int st)
 {
   if (st == 0)
-    return hydro3d_step<T, T3X, T3Y, N3T, RS, 0>;
+    return hydro3d_step<T, TX, TY, N3T, RS, 0>;
   if (st == 1)
-    return hydro3d_step<T, T3X, T3Y, N3T, RS, 1>;
-  return hydro3d_step<T, T3X, T3Y, N3T, RS, 2>;
+    return hydro3d_step<T, TX, TY, N3T, RS, 1>;
+  return hydro3d_step<T, TX, TY, N3T, RS, 2>;
+}
+template <class T, int TX, int TY>
+inline void launch3(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, const Gas<T>& gas, const StepCtl& ctl,
+                    int cz, hipStream_t s)
+{
+  Step3Fn<T> f;
+  switch (rs) {
+    case RS_APPROX: f = pick3<T, TX, TY, RS_APPROX>(st); break;
+    case RS_LLF: f = pick3<T, TX, TY, RS_LLF>(st); break;
+    default: f = pick3<T, TX, TY, RS_HLLC>(st); break;
+  }
+  const int ntx = (geo.nx + TX - 1) / TX, nty = (geo.ny + TY - 1) / TY, nch = (geo.nz + cz - 1) / cz;
+  hipLaunchKernelGGL(f, dim3(ntx * nty * nch), dim3(N3T), 0, s, Uin, Uout, geo, gas, ctl, cz, ntx, nty, nch);
 }
 
 template <class T>
@@ -75,17 +88,10 @@ inline hipError_t launch_step(int dim, int rs, int st, const T* Uin, T* Uout, co
       launch2<T, SmallTile2>(rs, st, Uin, Uout, geo, gas, ctl, s);
     else
       launch2<T, Tile2Of<T>>(rs, st, Uin, Uout, geo, gas, ctl, s);
+  } else if (cz < 0) { // hydro3d_z_chunk's sign
+    launch3<T, T3Y, T3X>(rs, st, Uin, Uout, geo, gas, ctl, -cz, s);
   } else {
-    Step3Fn<T> f;
-    switch (rs) {
-      case RS_APPROX: f = pick3<T, RS_APPROX>(st); break;
-      case RS_LLF: f = pick3<T, RS_LLF>(st); break;
-      default: f = pick3<T, RS_HLLC>(st); break;
-    }
-    const int ntx = (geo.nx + T3X - 1) / T3X, nty = (geo.ny + T3Y - 1) / T3Y;
-    const int nch = (geo.nz + cz - 1) / cz;
-    hipLaunchKernelGGL(f, dim3(ntx * nty * nch), dim3(N3T), 0, s, Uin, Uout, geo, gas, ctl, cz, ntx,
-                       nty, nch);
+    launch3<T, T3X, T3Y>(rs, st, Uin, Uout, geo, gas, ctl, cz, s);
   }
   return hipGetLastError();
 }
