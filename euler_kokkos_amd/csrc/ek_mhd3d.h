@@ -3,7 +3,7 @@
 // One step is SolverMHDMuscl<3>::godunov_unsplit_impl, impl 0 (src/muscl/SolverMHDMuscl.cpp:
 // 462-512), as a pipeline of kernels over a ghost-padded SoA work area (x fastest, 3 ghost
 // layers each side, so padded index (i,j,k) is the reference's U(i,j,k)):
-//   padprims: interior state -> padded state, ghosts through the boundary map, and the
+//   padprims: interior state -> padded face fields, ghosts through the boundary map, and the
 //             primitives with the right/top/front face fields (ConvertToPrimitivesFunctor3D_MHD)
 //   efield  : edge electric fields (ComputeElecFieldFunctor3D)
 //   fluxemf : the half-step record of every cell (trace_unsplit_mhd_3d_simpler) in LDS: centred
@@ -33,12 +33,12 @@ struct Work3 {
 
 // offsets (in arrays of PN elements) inside the scratch block
 enum {
-  A_UP = 0,           // padded state, 8
-  A_Q = 8,            // primitives, 8
-  A_E = 16,           // Ex, Ey, Ez
-  A_FLUX = 19,        // Fx, Fy, Fz: 3 x 5 (ID IP IU IV IW of the update, unrotated)
-  A_EMF = 34,         // EMF x, y, z
-  A_TOTAL = 37
+  A_B = 0,            // padded face fields IA, IB, IC (A_B + v - IA)
+  A_Q = 3,            // primitives, 8
+  A_E = 11,           // Ex, Ey, Ez
+  A_FLUX = 14,        // Fx, Fy, Fz: 3 x 5 (ID IP IU IV IW of the update, unrotated)
+  A_EMF = 29,         // EMF x, y, z
+  A_TOTAL = 32
 };
 
 // Half-step record of a cell: K_C + v the centred state (component order of the state),
@@ -135,7 +135,7 @@ __device__ __forceinline__ bool step_dt(const StepCtl& c, double& dt)
   return true;
 }
 
-// pad + prims in one pass. The padded state: ghost values as SolverBase::make_boundaries
+// pad + prims in one pass. The padded face fields: ghost values as SolverBase::make_boundaries
 // fills them (X, then Y, then Z passes; reflecting axes negate the normal momentum and the
 // normal face field). On i < PX-1, j < PY-1, k < PZ-1 also the primitives
 // (ConvertToPrimitivesFunctor3D_MHD), whose right / top / front face fields are the padded
@@ -157,7 +157,8 @@ __device__ __forceinline__ void padprims_cell(const T* __restrict__ U, T* __rest
     T x = U[v * vs + o];
     if ((fx && (v == IU || v == IA)) || (fy && (v == IV || v == IB)) || (fz && (v == IW || v == IC)))
       x = x * T(-1);
-    S[(A_UP + v) * PN + po] = x;
+    if (v >= IA)
+      S[(A_B + v - IA) * PN + po] = x;
     u[v] = x;
   }
   if (i >= w.PX - 1 || j >= w.PY - 1 || k >= w.PZ - 1)
@@ -206,9 +207,9 @@ __device__ __forceinline__ void efield_cell(T* __restrict__ S, const Work3& w, i
   const long long PN = w.PN, o = pidx(w, i, j, k);
   const long long sx = 1, sy = w.PX, sz = (long long)w.PX * w.PY;
   const T* Q = S + A_Q * PN;
-  const T* Up = S + A_UP * PN;
+  const T* Bp = S + A_B * PN;
   auto q = [&](int v, long long off) -> T { return Q[v * PN + o + off]; };
-  auto u = [&](int v, long long off) -> T { return Up[v * PN + o + off]; };
+  auto u = [&](int v, long long off) -> T { return Bp[(v - IA) * PN + o + off]; };
   T vv, ww, uu, A, B, C;
   vv = T(0.25) * (q(IV, -sy - sz) + q(IV, -sy) + q(IV, -sz) + q(IV, 0));
   ww = T(0.25) * (q(IW, -sy - sz) + q(IW, -sy) + q(IW, -sz) + q(IW, 0));
@@ -480,7 +481,7 @@ __device__ __forceinline__ void record_to_lds(const T* __restrict__ S, const Wor
   const unsigned o = pidx(w, i, j, k) * (unsigned)sizeof(T), sx = sizeof(T), sy = (unsigned)w.PX * (unsigned)sizeof(T);
   const unsigned sz = (unsigned)(w.PX * w.PY) * (unsigned)sizeof(T);
   auto q = [&](int v, unsigned off) { return ldb(S + (A_Q + v) * PN, off); };
-  auto u = [&](int v, unsigned off) { return ldb(S + (A_UP + v) * PN, off); };
+  auto u = [&](int v, unsigned off) { return ldb(S + (A_B + v - IA) * PN, off); };
   auto E = [&](int v, unsigned off) { return ldb(S + (A_E + v) * PN, off); };
   TraceIn<T> in;
 #pragma unroll
@@ -715,7 +716,7 @@ __device__ __forceinline__ double cfl3(const Gas<T>& gas, const T* u, T mx, T my
 // Flux update, CT update and the CFL term of the new state of interior cell c
 // (UpdateFunctor3D_MHD + UpdateEmfFunctor3D + ComputeDtFunctor3D_MHD on the result).
 template <class T>
-__device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __restrict__ Uout, const Work3& w,
+__device__ __forceinline__ double update_cell(const T* __restrict__ Uin, const T* __restrict__ S, T* __restrict__ Uout, const Work3& w,
                                               const Geom<T>& geo, const Gas<T>& gas, T dtdx, T dtdy, T dtdz,
                                               long long c)
 {
@@ -733,7 +734,7 @@ __device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __rest
     T u[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++)
-      u[v] = at(A_UP + v, o);
+      u[v] = v < IA ? ldb(Uin + v * n, ob) : at(A_B + v - IA, o);
     constexpr int hv[5] = { ID, IP, IU, IV, IW };
 #pragma unroll
     for (int m = 0; m < 5; m++) {
@@ -762,7 +763,7 @@ __device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __rest
     T ar, bt, cf;
     if (ii + 1 < w.nx || geo.bc[1] == BC_PERIODIC) {
       const unsigned q = o + sx;
-      ar = at(A_UP + IA, q);
+      ar = at(A_B + IA - IA, q);
       ar += (EZ(q + sy) - EZ(q)) * dtdy;
       ar -= (EY(q + sz) - EY(q)) * dtdz;
     } else {
@@ -770,7 +771,7 @@ __device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __rest
     }
     if (jj + 1 < w.ny || geo.bc[3] == BC_PERIODIC) {
       const unsigned q = o + sy;
-      bt = at(A_UP + IB, q);
+      bt = at(A_B + IB - IA, q);
       bt -= (EZ(q + sx) - EZ(q)) * dtdx;
       bt += (EX(q + sz) - EX(q)) * dtdz;
     } else {
@@ -778,7 +779,7 @@ __device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __rest
     }
     if (kk + 1 < w.nz || geo.bc[5] == BC_PERIODIC) {
       const unsigned q = o + sz;
-      cf = at(A_UP + IC, q);
+      cf = at(A_B + IC - IA, q);
       cf += (EY(q + sx) - EY(q)) * dtdx;
       cf -= (EX(q + sy) - EX(q)) * dtdy;
     } else {
@@ -795,7 +796,7 @@ __device__ __forceinline__ double update_cell(const T* __restrict__ S, T* __rest
 constexpr unsigned MHD3_UPDATE_BLOCKS = 2048;
 
 template <class T>
-__global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ S, T* __restrict__ Uout, Work3 w,
+__global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ Uin, const T* __restrict__ S, T* __restrict__ Uout, Work3 w,
                                                      Geom<T> geo, Gas<T> gas, StepCtl ctl)
 {
   __shared__ double sred[4];
@@ -809,7 +810,7 @@ __global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ S, T*
   double local = 0.0;
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n;
        c += (long long)gridDim.x * blockDim.x) {
-    const double sv = update_cell<T>(S, Uout, w, geo, gas, dtdx, dtdy, dtdz, c);
+    const double sv = update_cell<T>(Uin, S, Uout, w, geo, gas, dtdx, dtdy, dtdz, c);
     local = (sv > local || !(sv == sv)) ? sv : local;
   }
   block_max_to<256>(invdt_word(ctl, (ctl.slot + 1) % 3, blockIdx.x), local, sred);

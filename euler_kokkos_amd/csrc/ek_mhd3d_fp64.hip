@@ -18,7 +18,7 @@ static hipError_t launch3(const double* Uin, double* Uout, double* S, const mhd3
   const mhd3::FluxGrid fg = mhd3::flux_grid(geo);
   hipLaunchKernelGGL((mhd3::fluxemf_kernel<double, RS, ST>), dim3(fg.ntx * fg.nty * fg.ntz), dim3(mhd3::FCN), 0, s, S, w, geo,
                      gas, ctl, fg.cz, fg.ntx, fg.nty);
-  hipLaunchKernelGGL(mhd3::update_kernel<double>, dim3(ni), dim3(256), 0, s, S, Uout, w, geo, gas, ctl);
+  hipLaunchKernelGGL(mhd3::update_kernel<double>, dim3(ni), dim3(256), 0, s, Uin, S, Uout, w, geo, gas, ctl);
   return hipGetLastError();
 }
 

@@ -131,7 +131,7 @@ __device__ __forceinline__ void pool_range(int nwork, int& w0, int& w1)
 // first unit keeps the job's time bookkeeping. (Contiguous ranges measured faster than
 // grid-strided units here: 0.78 against 0.88 ms per 128^3 FP32 job in a pool of 8.)
 template <class T>
-__global__ __launch_bounds__(256) void mhd3_pool_update(const T* __restrict__ W, T* __restrict__ Ub,
+__global__ __launch_bounds__(256) void mhd3_pool_update(const T* __restrict__ Ua, const T* __restrict__ W, T* __restrict__ Ub,
                                                         const PoolJobM<T>* __restrict__ jobs,
                                                         const PoolWork* __restrict__ work, int nwork, TimeSlot* ts,
                                                         int slot)
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void mhd3_pool_update(const T* __restrict__ W,
     const T dtdx = T(dt / J.geo.dx), dtdy = T(dt / J.geo.dy), dtdz = T(dt / J.geo.dz);
     const long long c = ((long long)it.tx * UNITS_U + r) * 256 + threadIdx.x;
     if (c < J.geo.vstride) {
-      const double sv = mhd3::update_cell<T>(W + J.woff, Ub + J.off, J.w, J.geo, J.gas, dtdx, dtdy, dtdz, c);
+      const double sv = mhd3::update_cell<T>(Ua + J.off, W + J.woff, Ub + J.off, J.w, J.geo, J.gas, dtdx, dtdy, dtdz, c);
       local = (sv > local || !(sv == sv)) ? sv : local;
     }
     if (first && threadIdx.x < 64)
@@ -197,7 +197,7 @@ inline hipError_t mhd3_launch(const T* Ua, T* Ub, T* W, const PoolJobM<T>* jobs,
   hipLaunchKernelGGL(mhd3_pool_efield<T>, dim3(UNITS_P * np), dim3(256), 0, s, W, jobs, wp, np, ts, slot);
   hipLaunchKernelGGL((mhd3_pool_fluxemf<T, RS, ST>), dim3(nf), dim3(mhd3::FCN), 0, s, W, jobs, wf, ts, slot);
   hipLaunchKernelGGL(mhd3_pool_update<T>, dim3((unsigned)(ugrid < UNITS_U * nu ? ugrid : UNITS_U * nu)), dim3(256), 0, s,
-                     W, Ub, jobs, wu, nu, ts, slot);
+                     Ua, W, Ub, jobs, wu, nu, ts, slot);
   return hipGetLastError();
 }
 
