@@ -112,7 +112,10 @@ __device__ __forceinline__ void split3(unsigned c, unsigned X, unsigned Y, int& 
 template <class T>
 __device__ __forceinline__ bool cell_of(const Work3& w, int& i, int& j, int& k)
 {
-  const unsigned c = blockIdx.x * blockDim.x + threadIdx.x;
+  // XCD order: the rows and planes a cell's neighbours are on were read on the same XCD (per step
+  // 64^3 FP64 126.4 -> 122.9 us, FP32 64.9 -> 63.9; 97x64x110 312 -> 307 and 149 -> 146; 128^3 FP64
+  // 897 -> 896, FP32 388 -> 382; the update in that order was up to 3 % slower)
+  const unsigned c = xcd_order(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (c >= (unsigned long long)w.PN)
     return false;
   split3(c, (unsigned)w.PX, (unsigned)w.PY, i, j, k);
