@@ -102,13 +102,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
   ctl.tEnd = J.tEnd;
   ctl.nStepmax = J.nStepmax;
   const bool first = (it.tz_first & 1) != 0;
-  double dt;
+  double dt, local;
   TimeSlot cur;
-  if (!step_begin(ctl, first, dt, cur))
+  auto begin = [&](double& d) {
+    const bool go = step_begin(ctl, first, dt, cur);
+    d = dt;
+    return go;
+  };
+  if (!hydro3d_column<T, TX, TY, NT, RS, ST, false>(Ua + J.off, Ub + J.off, J.geo, J.gas, begin, it.tx * TX,
+                                                    it.ty * TY, (it.tz_first >> 1) * J.cz, J.cz, local))
     return;
-  const double local = hydro3d_column<T, TX, TY, NT, RS, ST, false>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt,
-                                                             it.tx * TX, it.ty * TY, (it.tz_first >> 1) * J.cz,
-                                                             J.cz);
   block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
   if (first && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);
