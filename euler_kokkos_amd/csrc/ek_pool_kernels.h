@@ -80,8 +80,7 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
 }
 
 // Occupancy targets: FP64 3 waves per SIMD (what the shared memory allows anyway); FP32 5,
-// which its shared memory also allows: the compiler would otherwise keep 119 registers (4
-// waves); at 96 it spills 12 and runs a serving burst of 3D jobs 7 % faster.
+// which its shared memory also allows (93 registers, no spills).
 template <class T, int TX, int TY, int NT, int RS, int ST>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 5))) void hydro3d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
