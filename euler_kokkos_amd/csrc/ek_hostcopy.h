@@ -38,13 +38,14 @@ inline void in_parts(long long n, long long grain, F work)
     th[t].join();
 }
 
-// Whether there are page faults to be taken in [mem, mem + bytes): not in pinned memory, nor where
-// a page at each eighth of it is in memory.
+// Whether there are page faults to be taken in [mem, mem + bytes): not in memory the runtime knows
+// (pinned, or the device's: no page of the host's to touch), nor where a page at each eighth of it
+// is in memory.
 inline bool faults(const char* mem, long long bytes)
 {
   hipPointerAttribute_t at;
   const hipError_t e = hipPointerGetAttributes(&at, mem);
-  if (e == hipSuccess && at.type == hipMemoryTypeHost)
+  if (e == hipSuccess && at.type != hipMemoryTypeUnregistered)
     return false;
   if (e != hipSuccess)
     (void)hipGetLastError(); // memory that the runtime does not know

@@ -1,6 +1,7 @@
 """Host side of the downloads (csrc/ek_hostcopy.h) with the device copy replaced by a stub: a copy
 that fails leaves the destination as it was, whether its pages are in memory or not, and one that
-succeeds fills it (FP32 widened), at sizes of one part, of two and of the most."""
+succeeds fills it (FP32 widened), at sizes of one part, of two and of the most. A destination that
+is device memory is the copy's alone to write."""
 import os
 import shutil
 import subprocess
@@ -19,6 +20,7 @@ DRIVER = r"""
 #include <sys/mman.h>
 
 static bool fails;
+static const void* device; // stands for device memory: no access from the host
 extern "C" hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t)
 {
   if (fails)
@@ -27,7 +29,11 @@ extern "C" hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMe
   return hipSuccess;
 }
 extern "C" hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-extern "C" hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) { return hipErrorInvalidValue; }
+extern "C" hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+  a->type = hipMemoryTypeDevice;
+  return p == device ? hipSuccess : hipErrorInvalidValue;
+}
 extern "C" hipError_t hipGetLastError() { return hipErrorInvalidValue; }
 
 int main()
@@ -59,6 +65,12 @@ int main()
         }
         munmap(host, n * 8);
       }
+  for (long long n : { 1000LL, 8388608LL + 1 }) {
+    std::vector<double> s64(n);
+    device = mmap(nullptr, n * 8, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+    fails = true; // the stub has no way to write there either
+    bad += ek::copy_to_host((double*)device, s64.data(), false, n, nullptr) == hipSuccess;
+  }
   printf("%d bad\n", bad);
   return bad != 0;
 }
