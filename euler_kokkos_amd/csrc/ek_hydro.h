@@ -39,6 +39,7 @@ struct StepCtl {
   double cfl;
   double tEnd;
   int nStepmax;
+  unsigned tile0;  // 2D steps: first tile of this launch (in_launches)
 };
 
 template <class T>
@@ -220,6 +221,17 @@ __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
 {
   const unsigned n8 = n / 8;
   return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;
+}
+
+// A launch takes fewer than 2^32 threads (more are refused by one way of launching and cut off
+// without an error by another), and a 2D state of 137 GB can have that many: launch(first, count)
+// for parts of `blocks` blocks of nt threads.
+template <class F>
+inline void in_launches(long long blocks, int nt, F launch)
+{
+  const long long most = ((1LL << 32) - 1) / nt;
+  for (long long b = 0; b < blocks; b += most)
+    launch((unsigned)b, (unsigned)(blocks - b < most ? blocks - b : most));
 }
 
 // Planes per z-chunk of a launch of `tiles` column tiles over n planes: a block marches over its
@@ -580,8 +592,8 @@ __global__ __launch_bounds__(NT) void hydro2d_step(const T* __restrict__ Uin, T*
                                                    Geom<T> geo, Gas<T> gas, StepCtl ctl)
 {
   __shared__ double sred[NT / 64];
-  const bool first_block = blockIdx.x == 0;
-  const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(geo.nx + TX - 1) / TX;
+  const bool first_block = blockIdx.x == 0 && ctl.tile0 == 0;
+  const unsigned tile = ctl.tile0 + xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(geo.nx + TX - 1) / TX;
   const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
   Loaded2<T, TX, TY, NT> in;
   hydro2d_load<T, TX, TY, NT>(Uin, geo, i0, j0, in);

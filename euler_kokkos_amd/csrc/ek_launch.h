@@ -53,8 +53,12 @@ inline void launch2(int rs, int st, const T* Uin, T* Uout, const Geom<T>& geo, c
     case RS_HLL: f = pick2<T, C, RS_HLL>(st); break;
     default: f = pick2<T, C, RS_HLLC>(st); break;
   }
-  dim3 grid((unsigned)((geo.nx + C::X - 1) / C::X) * (unsigned)((geo.ny + C::Y - 1) / C::Y));
-  hipLaunchKernelGGL(f, grid, dim3(C::NT), 0, s, Uin, Uout, geo, gas, ctl);
+  const long long blocks = (long long)((geo.nx + C::X - 1) / C::X) * ((geo.ny + C::Y - 1) / C::Y);
+  StepCtl part = ctl;
+  in_launches(blocks, C::NT, [&](unsigned first, unsigned count) {
+    part.tile0 = first;
+    hipLaunchKernelGGL(f, dim3(count), dim3(C::NT), 0, s, Uin, Uout, geo, gas, part);
+  });
 }
 template <class T, int TX, int TY, int RS>
 inline Step3Fn<T> pick3(int st)

@@ -588,10 +588,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, WPE))) vo
   T* const sDBx = sBev + L::BYN;         // [BYN] transverse slope dB/dx at y faces (halved)
 
   const int tid = threadIdx.x;
-  const bool first_block = blockIdx.x == 0;
+  const bool first_block = blockIdx.x == 0 && ctl.tile0 == 0;
   const int nx = geo.nx, ny = geo.ny;
   const long long vs = geo.vstride;
-  const unsigned tile = xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(nx + TX - 1) / TX;
+  const unsigned tile = ctl.tile0 + xcd_order(blockIdx.x, gridDim.x), ntx = (unsigned)(nx + TX - 1) / TX;
   const int i0 = (int)(tile % ntx) * TX, j0 = (int)(tile / ntx) * TY;
 
   // A: primitives and raw face fields on cells -2..TX+1 (ghosts through the boundary map;

@@ -67,7 +67,11 @@ inline void launch_tiles(int rs, int st, const T* Uin, T* Uout, const Geom<T>& g
     case RS_LLF: f = pick<T, M, RS_LLF>(st); break;
     default: f = pick<T, M, RS_HLLD>(st); break;
   }
-  hipLaunchKernelGGL(f, dim3((unsigned)blocks_of<M>(geo)), dim3(M::NT), 0, s, Uin, Uout, geo, gas, ctl);
+  StepCtl part = ctl;
+  in_launches(blocks_of<M>(geo), M::NT, [&](unsigned first, unsigned count) {
+    part.tile0 = first;
+    hipLaunchKernelGGL(f, dim3(count), dim3(M::NT), 0, s, Uin, Uout, geo, gas, part);
+  });
 }
 
 template <class T>

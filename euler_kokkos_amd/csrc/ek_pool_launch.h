@@ -71,11 +71,11 @@ inline hipError_t launch_step(int dim, int variant, int st, const T* Ua, T* Ub, 
 {
   if (nwork <= 0)
     return hipSuccess;
-  if (dim == 2)
-    hipLaunchKernelGGL(pick2<T>(variant, st), dim3(nwork), dim3(pool_tile2<T>(variant).nt), 0, s, Ua, Ub, jobs, work, ts,
-                       slot);
-  else
-    hipLaunchKernelGGL(pick3<T>(st), dim3(nwork), dim3(P3T), 0, s, Ua, Ub, jobs, work, ts, slot);
+  const Pool2Fn<T> f = dim == 2 ? pick2<T>(variant, st) : pick3<T>(st);
+  const int nt = dim == 2 ? pool_tile2<T>(variant).nt : P3T;
+  in_launches(nwork, nt, [&](unsigned first, unsigned count) {
+    hipLaunchKernelGGL(f, dim3(count), dim3(nt), 0, s, Ua, Ub, jobs, work + first, ts, slot);
+  });
   return hipGetLastError();
 }
 
