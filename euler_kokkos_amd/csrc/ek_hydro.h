@@ -217,7 +217,7 @@ __device__ __forceinline__ unsigned long long* reduce_word(unsigned long long* d
 // in this one, with 16x16 hydro and 14x14 or 30x14 MHD tiles: 2D hydro 64^2 9.6 -> 9.4 us,
 // 512^2 19.8 -> 18.2, 1000x333 FP32 two-shock 18.5 -> 14.6; 2D MHD 300x211 26.0 -> 22.8, 1024^2
 // 210 -> 206, FP32 84.1 -> 81.9).
-__device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
+__host__ __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n)
 {
   const unsigned n8 = n / 8;
   return b < n8 * 8 ? (b % 8) * n8 + b / 8 : b;

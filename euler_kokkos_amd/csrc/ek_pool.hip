@@ -38,8 +38,8 @@ struct HostJob {
 
 constexpr long long kAlign = 64; // elements
 constexpr int kGraphSteps = 6;   // lcm of the 2 arena buffers and the 3 time slots
-// job slots with their own spread CFL words (12 KiB each); a pool with more jobs than this has
-// so many tiles of other jobs in flight that one word per job is enough for the rest
+// job slots with their own spread CFL words (24 KiB each), which bounds them to 48 MiB; the jobs in
+// further slots have one word each (and queue on it: 546 against 289 us, ek_pool_kernels.h)
 constexpr int kSpreadJobs = 2048;
 constexpr int kCz[4] = { 8, 16, 32, 64 };
 // 3D MHD pools: share of the arena for the two state buffers; the rest is the work buffer
@@ -1154,6 +1154,15 @@ extern "C" int ek_pool_autotune(ek_pool* p, int steps, int* choice, double* ms_o
     return rc;
   if (choice)
     *choice = bestv;
+  return EK_OK;
+}
+
+extern "C" int ek_pool_test_item(unsigned block, unsigned blocks, unsigned* item, unsigned* word)
+{
+  if (block >= blocks || !item || !word)
+    return EK_EINVAL;
+  *item = ek::pool_item(block, blocks);
+  *word = ek::pool_word(block);
   return EK_OK;
 }
 

@@ -10,12 +10,11 @@
 //
 // A tile is short and starts with a chain of dependent reads (item, job record, time slot, CFL
 // words, cells), so what counts is how many tiles are in flight and how long their closing
-// atomics queue. One word per job made the atomics of a job's tiles serialize (about 70 ns
-// each): 24 blasts of edges 64-320 took 57 us per step, 256 of edges 64-512 682 us (FP32), 100
-// of them 564 us (FP64) in a persistent grid walking ranges of the list. With 16 words per job
-// (4 to 64 measured alike but for 64's longer reads), one block per item and the items in
-// XCD order (33 us without it): 30, 617 and 496 us. 3D jobs (six of edges 64-160): 452 -> 324 us
-// FP32, 898 -> 709 us FP64.
+// atomics queue: on one word per job they serialize (about 70 ns each). us per step in a persistent
+// grid walking ranges of the list with one word per job -> with one block per item, the items in
+// XCD order and 32 words per job: 24 blasts of edges 64-320 60 -> 29 FP32, 72 -> 46 FP64; 128 of
+// edges 64-512 FP32 372 -> 289; 64 of them FP64 402 -> 245; 3D jobs (six of edges 64-128) 278 -> 201
+// and 606 -> 484. Figures for other numbers of words beside pool_word.
 #pragma once
 
 #include "ek_hydro.h"
@@ -24,7 +23,7 @@
 namespace ek {
 
 // CFL words per slot of a job
-constexpr int POOL_NSPREAD = 16;
+constexpr int POOL_NSPREAD = 32;
 constexpr long long POOL_SPREAD_ELEMS = 3LL * POOL_NSPREAD * SPREAD_STRIDE;
 
 template <class T>
@@ -46,6 +45,21 @@ struct PoolWork {
   int tz_first; // z chunk * 2 + (1 if this item does the job's bookkeeping)
 };
 
+// Position in the work list of the item that block b of n runs, and which of its job's CFL words
+// takes its term: words in turn both along an XCD's blocks (8 apart in b, one item of the list
+// after another, and so one job's for many blocks) and across the XCDs (where a job that fills the
+// launch runs on all of them at once). us per step, 1 / 4 / 8 / 16 / 32 / 64 words, FP32: 128 jobs of
+// edges 64-512 546, 310, 292, 290, 289, 288; 24 of edges 64-320 48, 30, 29, 28, 29, 28; one of 1024^2
+// 150, 74, 56, 42, 33, 30; one of 512^2 (16 words and more) 10.7, 10.8, 10.8; in FP64 64's longer
+// reads show (six 3D jobs 484, 484, 484, 484, 484, 486). By block number alone the items of a job
+// that run side by side on one XCD meet on two of 16 words: 128 jobs 326 to 378, one of 1024^2 35 to
+// 41, one of 512^2 10.3.
+__host__ __device__ __forceinline__ unsigned pool_item(unsigned b, unsigned n) { return xcd_order(b, n); }
+__host__ __device__ __forceinline__ unsigned pool_word(unsigned b)
+{
+  return (b / 8 + b % 8 * (POOL_NSPREAD / 8)) & (unsigned)(POOL_NSPREAD - 1);
+}
+
 template <class T, int TX, int TY, int NT, int RS, int ST, bool CMP>
 __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua, T* __restrict__ Ub,
                                                         const PoolJob<T>* __restrict__ jobs,
@@ -53,7 +67,7 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  const PoolWork it = work[xcd_order(blockIdx.x, gridDim.x)];
+  const PoolWork it = work[pool_item(blockIdx.x, gridDim.x)];
   const PoolJob<T> J = jobs[it.job];
   StepCtl ctl;
   ctl.ts = ts + J.slot0;
@@ -74,7 +88,7 @@ __global__ __launch_bounds__(NT) void hydro2d_pool_step(const T* __restrict__ Ua
     return;
   const double local =
       hydro2d_tile<T, TX, TY, NT, RS, ST, CMP>(Ua + J.off, Ub + J.off, J.geo, J.gas, dt, it.tx * TX, it.ty * TY, in);
-  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
+  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, pool_word(blockIdx.x)), local, sred);
   if (first && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);
 }
@@ -88,7 +102,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
                                                         TimeSlot* ts, int slot)
 {
   __shared__ double sred[NT / 64];
-  const PoolWork it = work[xcd_order(blockIdx.x, gridDim.x)];
+  const PoolWork it = work[pool_item(blockIdx.x, gridDim.x)];
   const PoolJob<T> J = jobs[it.job];
   StepCtl ctl;
   ctl.ts = ts + J.slot0;
@@ -111,7 +125,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
   if (!hydro3d_column<T, TX, TY, NT, RS, ST, false>(Ua + J.off, Ub + J.off, J.geo, J.gas, begin, it.tx * TX,
                                                     it.ty * TY, (it.tz_first >> 1) * J.cz, J.cz, local))
     return;
-  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, blockIdx.x), local, sred);
+  block_max_to<NT>(invdt_word(ctl, (slot + 1) % 3, pool_word(blockIdx.x)), local, sred);
   if (first && threadIdx.x < 64)
     step_end_bookkeeping(ctl, cur, dt);
 }

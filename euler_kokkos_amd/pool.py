@@ -27,7 +27,7 @@ POOL_EXPORTS = ("ek_pool_create", "ek_pool_destroy", "ek_pool_last_error", "ek_p
                 "ek_pool_free_bytes", "ek_pool_active", "ek_pool_admit", "ek_pool_step",
                 "ek_pool_status", "ek_pool_download", "ek_pool_budgets", "ek_pool_retire",
                 "ek_pool_autotune", "ek_pool_set_tile", "ek_pool_last_step_time", "ek_pool_test_fail_admit",
-                "ek_pool_admit_async", "ek_pool_test_defer_join")
+                "ek_pool_admit_async", "ek_pool_test_defer_join", "ek_pool_test_item")
 
 _BOUND = False
 
@@ -60,6 +60,7 @@ def _lib() -> C.CDLL:
         L.ek_pool_last_step_time.argtypes = [V, D, P(C.c_int)]
         L.ek_pool_test_fail_admit.argtypes = [V, C.c_int]
         L.ek_pool_test_defer_join.argtypes = [V, C.c_int]
+        L.ek_pool_test_item.argtypes = [C.c_uint, C.c_uint, P(C.c_uint), P(C.c_uint)]
         _BOUND = True
     return L
 

@@ -102,6 +102,10 @@ int ek_pool_test_fail_admit(ek_pool* pool, int stage);
  * are stepping (so that tests can make it join after an odd number of steps); 0 turns it off. */
 int ek_pool_test_defer_join(ek_pool* pool, int calls);
 
+/* Test hook: which item of the work list block `block` of a hydro pool launch of `blocks` blocks
+ * runs, and which of its job's 32 CFL words it updates. */
+int ek_pool_test_item(unsigned block, unsigned blocks, unsigned* item, unsigned* word);
+
 #ifdef __cplusplus
 }
 #endif
