@@ -4,10 +4,12 @@
 #include "ek_internal.h"
 #include "ek_geom_host.h"
 #include "ek_hostcopy.h"
+#include "ek_mhd3d.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -174,6 +176,34 @@ static int z_chunk(const ek_params* p)
     return 1;
   return p->precision == EK_FP64 ? ek::hydro3d_z_chunk<double>(p->nx, p->ny, p->nz)
                                  : ek::hydro3d_z_chunk<float>(p->nx, p->ny, p->nz);
+}
+
+extern "C" int ek_test_z_chunk(const ek_params* params, int* planes, int* tile_x, int* tile_y)
+{
+  std::string why;
+  if (!params || !planes || !tile_x || !tile_y)
+    return fail(nullptr, EK_EINVAL, "null argument");
+  if (ek::validate_params(params, why))
+    return fail(nullptr, EK_EINVAL, why);
+  if (params->dim != 3)
+    return fail(nullptr, EK_EINVAL, "dim must be 3");
+  if (params->mhd) {
+    ek::Geom<double> g64;
+    ek::Gas<double> gas64;
+    ek::Geom<float> g32;
+    ek::Gas<float> gas32;
+    ek::fill_geom<double>(*params, g64, gas64);
+    ek::fill_geom<float>(*params, g32, gas32);
+    *planes = (params->precision == EK_FP64 ? ek::mhd3::flux_grid(g64) : ek::mhd3::flux_grid(g32)).cz;
+    *tile_x = ek::mhd3::FCX;
+    *tile_y = ek::mhd3::FCY;
+  } else {
+    const int cz = z_chunk(params);
+    *planes = std::abs(cz);
+    *tile_x = cz < 0 ? ek::T3Y : ek::T3X;
+    *tile_y = cz < 0 ? ek::T3X : ek::T3Y;
+  }
+  return EK_OK;
 }
 
 extern "C" int ek_create(const ek_params* params, ek_ctx** out)

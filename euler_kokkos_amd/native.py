@@ -21,7 +21,7 @@ RIEMANN = {"approx": 0, "llf": 1, "hll": 2, "hllc": 3, "hlld": 4}
 # Exported symbols declared by include/ek_hip.h (checked by the CPU test-suite).
 EXPORTS = ("ek_create", "ek_destroy", "ek_last_error", "ek_upload", "ek_download", "ek_inv_dt",
            "ek_step", "ek_run", "ek_budgets", "ek_sync", "ek_device_bytes", "ek_last_run_time",
-           "ek_host_alloc", "ek_host_free", "ek_device_info", "ek_run_noalloc")
+           "ek_host_alloc", "ek_host_free", "ek_device_info", "ek_run_noalloc", "ek_test_z_chunk")
 # size of the fixed device array behind ek_run_noalloc (EK_NOALLOC_SCRATCH_BYTES)
 NOALLOC_SCRATCH_BYTES = 16 << 20
 
@@ -77,6 +77,8 @@ def lib() -> C.CDLL:
     L.ek_device_info.argtypes = [P(C.c_int), P(C.c_int), P(C.c_int), P(C.c_int), C.c_char_p, C.c_int]
     L.ek_run_noalloc.argtypes = [P(EkParams), C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_double,
                                  P(C.c_double), P(C.c_int), P(C.c_double), P(C.c_int), C.c_void_p]
+    L.ek_test_z_chunk.argtypes = [P(EkParams), P(C.c_int), P(C.c_int), P(C.c_int)]
+    L.ek_test_z_chunk.restype = C.c_int
     for n in ("ek_upload", "ek_download", "ek_inv_dt", "ek_step", "ek_run", "ek_budgets", "ek_sync",
               "ek_host_alloc", "ek_host_free", "ek_device_info", "ek_run_noalloc"):
         getattr(L, n).restype = C.c_int
@@ -94,6 +96,15 @@ def device_info() -> dict:
         raise EkError(f"ek_device_info failed ({rc})")
     return {"cus": cus.value, "mem_clock_khz": mclk.value, "bus_width_bits": bw.value,
             "sclk_khz": sclk.value, "name": name.value.decode(errors="replace")}
+
+
+def z_chunk(params: EkParams):
+    """(planes per z-chunk, tile cells along x, along y) of a 3D step (ek_test_z_chunk)."""
+    v = [C.c_int() for _ in range(3)]
+    rc = lib().ek_test_z_chunk(C.byref(params), *[C.byref(x) for x in v])
+    if rc != 0:
+        raise EkError(f"ek_test_z_chunk failed ({rc}): {lib().ek_last_error(None).decode()}")
+    return tuple(x.value for x in v)
 
 
 def run_noalloc(params: EkParams, U: int, U2: int, nsteps: int, nStepmax: int, tEnd: float,

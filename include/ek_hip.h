@@ -156,6 +156,10 @@ int ek_host_free(void* ptr);
  * counterpart: measurement support.) */
 int ek_device_info(int* cus, int* mem_clock_khz, int* bus_width_bits, int* sclk_khz, char* name, int name_len);
 
+/* Test hook: the column tile (cells along x and y) and the planes per z-chunk that a 3D step of these
+ * parameters is launched with (3D MHD: its flux/EMF kernel). Host only, no device call. */
+int ek_test_z_chunk(const ek_params* params, int* planes, int* tile_x, int* tile_y);
+
 #ifdef __cplusplus
 }
 #endif
