@@ -26,7 +26,7 @@ struct HostJob {
   long long join_after = 0; // no earlier than this ek_pool_step call (ek_pool_test_defer_join)
   ek_params p{};
   long long off = 0, nelem = 0, alloc = 0;
-  long long woff = 0, walloc = 0; // 3D MHD: the job's padded work area in the work buffer
+  long long woff = 0, walloc = 0; // 3D MHD: the job's padded work area, as counted (kWorkPart)
   long long adm_step = 0;
   int nStepmax = 0;
   double tEnd = 0.0;
@@ -42,9 +42,13 @@ constexpr int kGraphSteps = 6;   // lcm of the 2 arena buffers and the 3 time sl
 // further slots have one word each (and queue on it: 546 against 289 us, ek_pool_kernels.h)
 constexpr int kSpreadJobs = 2048;
 constexpr int kCz[4] = { 8, 16, 32, 64 };
-// 3D MHD pools: share of the arena for the two state buffers; the rest is the work buffer
-// (78 reals per ghost-padded cell against 2 x 8 per cell: 13-16 % for edges 64-192)
+// 3D MHD pools: share of the arena for the two state buffers; the rest counts for the work areas
+// (78 reals per ghost-padded cell against 2 x 8 per cell: 13-16 % for edges 64-192). The pipeline
+// uses 32 of the 78, and the work buffer holds memory for half of what is counted: a job's area
+// starts at half its counted offset (a multiple of 32 reals).
 constexpr double kMhdStateShare = 0.16;
+constexpr int kWorkPart = 2;
+static_assert(kWorkPart * ek::mhd3::A_TOTAL <= ek::kMhd3LimitReals, "a job's work area fits its part of the buffer");
 
 long long round_up(long long n)
 {
@@ -190,7 +194,7 @@ static ek::PoolJobM<T> make_record_m(const ek_pool* p, int id)
   const HostJob& h = p->jobs[id];
   ek::PoolJobM<T> r{};
   r.off = h.off;
-  r.woff = h.woff;
+  r.woff = h.woff / kWorkPart;
   r.slot0 = 3 * id;
   r.nStepmax = h.nStepmax;
   r.cfl = h.p.cfl;
@@ -531,7 +535,7 @@ extern "C" int ek_pool_create(const ek_params* kind, long long arena_bytes, int 
       (e = hipStreamCreateWithFlags(&p->ustream, hipStreamNonBlocking)) != hipSuccess ||
       (e = hipMalloc(&p->A[0], (size_t)p->cap * p->elem)) != hipSuccess ||
       (e = hipMalloc(&p->A[1], (size_t)p->cap * p->elem)) != hipSuccess ||
-      (mhd3 && (e = hipMalloc(&p->W, (size_t)p->wcap * p->elem)) != hipSuccess) ||
+      (mhd3 && (e = hipMalloc(&p->W, (size_t)(p->wcap / kWorkPart) * p->elem)) != hipSuccess) ||
       (e = hipMalloc(&p->ts, (size_t)max_jobs * 3 * sizeof(ek::TimeSlot))) != hipSuccess ||
       (e = hipMalloc(&p->djobs, (size_t)max_jobs * recb)) != hipSuccess ||
       (spread_bytes(p) && (e = hipMalloc(&p->spread, spread_bytes(p))) != hipSuccess) ||

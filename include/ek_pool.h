@@ -13,9 +13,10 @@
  * job by one step of its own dt, one block per (job, tile) item of a work
  * list; consecutive steps over an unchanged job set are replayed from a
  * captured HIP graph. Tile shapes are chosen by ek_pool_autotune. A 3D MHD pool also keeps
- * each job's ghost-padded work area (78 reals per padded cell) in a work buffer that takes
- * 84 % of arena_bytes (the two state buffers take the rest), and one pool step is the four
- * kernels of the 3D MHD step, each over all active jobs.
+ * each job's ghost-padded work area, counted as 78 reals per padded cell against 84 % of
+ * arena_bytes (the two state buffers count for the rest; the areas need less than is counted, and
+ * the pool holds 58 % of arena_bytes), and one pool step is the four kernels of the 3D MHD step,
+ * each over all active jobs.
  *
  * All calls return 0 or an EK_E* code (include/ek_hip.h) with a message from
  * ek_pool_last_error. One pool per host thread.
@@ -37,7 +38,8 @@ typedef struct ek_pool ek_pool;
  * precision are taken from it (grid sizes, boundaries and constants may differ per job).
  * Supported: hydro 2D and 3D with HLLC, and 3D MHD with HLLD, HLL or LLF; slope_type 1 or 2;
  * FP64 or FP32.
- * arena_bytes: device bytes for job states (split over the two ping-pong buffers). */
+ * arena_bytes: device bytes for job states (split over the two ping-pong buffers), and for 3D MHD
+ * their work areas. */
 int ek_pool_create(const ek_params* kind, long long arena_bytes, int max_jobs, ek_pool** out);
 void ek_pool_destroy(ek_pool* pool);
 const char* ek_pool_last_error(const ek_pool* pool);
