@@ -244,13 +244,11 @@ inline int z_chunk_of(long long tiles, int n, int slots, double a, double b, int
 {
   int best = n < hi ? n : hi;
   double least = 1e300;
-  for (int nch = 1; nch <= n; nch++) {
-    const int cz = (n + nch - 1) / nch;
-    if (cz > hi)
-      continue;
-    if (cz < lo)
-      break;
-    const long long m = tiles * ((n + cz - 1) / cz), rest = m % slots;
+  for (int cz = best; cz >= lo; cz--) {
+    const int nch = (n + cz - 1) / cz;
+    if ((n + nch - 1) / nch != cz)
+      continue; // as many shorter chunks do
+    const long long m = tiles * nch, rest = m % slots;
     const double rounds = (double)(m / slots) + (rest ? b + (1.0 - b) * (double)rest / slots : 0.0);
     if ((cz + a) * rounds < least) {
       least = (cz + a) * rounds;
