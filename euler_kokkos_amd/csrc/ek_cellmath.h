@@ -3,7 +3,8 @@
 // Every function keeps the reference's floating-point operation order exactly (no
 // reassociation; divisions by one denominator share its reciprocal, each quotient still
 // rounded as the division rounds it), so that the FP64 build, compiled with
-// -ffp-contract=off, reproduces the reference's CPU results bit for bit. Shared
+// -ffp-contract=off, reproduces the reference's CPU results bit for bit (over the range that
+// quot states). Shared
 // subexpressions are computed once only where they are literally the same IEEE
 // expression in the reference (e.g. HALF*drx used by both faces of a cell).
 // Paths cited are relative to the euler_kokkos source tree.
@@ -54,10 +55,17 @@ __device__ __forceinline__ bool signbit_of(float a) { return __float_as_int(a) <
 // that scale with a density, a pressure or a speed, or whose quotient only enters a sum or
 // a comparison with such a term. quot_any takes any |a| < 2^895 (velocities, transverse
 // momenta and field components, which can be as small as they like in nearly quiet gas):
-// it forms the residual 2^128 times larger, one product more.
+// it forms the residual 2^128 times larger, one product more. A division, which scales its
+// operands as it needs, has no such limits. Below them a last bit can be off (quot_any: the
+// smallest denormal or zero), or more where the denominator is denormal; above them (quot_any: |a|
+// or |b| of 2^895 = 2.6e269 and more) the result is NaN. The numerators are products of at most
+// four speeds with a density or a field: with densities, pressures and squared fields from 1e-60
+// to 1e60 none comes near either end. Compared with a / b on 2.6e10 random operands and as many
+// with mantissas near powers of two: no bit differs.
 // FP32: the hardware reciprocal (1 ulp) and a product, two instructions where the compiler's
-// division has six (it scales denominators above 2^96). The product is rounded by itself
-// (plain): fused into the sum it enters, FP32 results would differ from a division's.
+// division has six. It scales denominators above 2^96; here one above 2^126, a density of 8.5e37,
+// has the reciprocal zero. The product is rounded by itself (plain): fused into the sum it enters,
+// FP32 results would differ from a division's.
 // With a division (and the library's root) everywhere, per step: 3D hydro 256^3 FP64 1.20 ms,
 // now 1.11, FP32 0.554 -> 0.531; 2D MHD 1024^2 FP64 0.250 -> 0.206, FP32 0.087 -> 0.078; 3D
 // MHD 128^3 FP64 1.34 -> 1.26 (same GPU, bitwise the same states; 3D MHD in FP32 is bound by
@@ -211,7 +219,10 @@ __device__ __forceinline__ T cell_inv_dt(const Gas<T>& g, const T* u, T dx, T dy
 // ST is slope_type (1 minmod, 2 MC); ST*x is written as the identical exact product.
 // In FP32 the limiter is two medians with zero (the median of x, y and 0 is their minmod;
 // |dcen| never is below the smaller one-sided difference, so ST 1 needs one): 7 instructions
-// where the comparisons take 13, the same values (3D hydro 256^3 0.587 -> 0.559 ms per step).
+// where the comparisons take 13 (3D hydro 256^3 0.587 -> 0.559 ms per step). The same values, but
+// for differences so small that their product underflows: there the comparisons see no common
+// sign and return 0, the medians the limited slope (gas of density 1e-6 and pressure 1e-18: 1e-2 of
+// the largest value off FP64 after three steps, 4e-7 to 1e-5 with the medians).
 template <class T, int ST>
 __device__ __forceinline__ T slope1(T q, T qp, T qm)
 {

@@ -4,7 +4,7 @@
 // position of the tile's (TX+4) x (TY+4) primitive grid for the whole march and keeps
 // that column's primitives at planes p-1, p, p+1 in registers, so the z slope never
 // touches LDS; only plane p (for the x/y slopes) and the face states live in LDS
-// (about 42 KB for 16x8 in FP64, three blocks per CU).
+// (53.5 KB for 16x8 in FP64, three blocks per CU).
 //
 // Per plane p:  A  load U(p+1), primitives into registers (all positions)
 //               B  slopes + Hancock trace at the tile and its 1-wide halo cross;

@@ -489,8 +489,9 @@ __device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
   const T AstarB = quot_any(SAR * AstarRL - SAL * AstarLL, iw);
   const T BstarR = quot_any(SAT * BstarRR - SAB * BstarRL, ih);
   const T BstarL = quot_any(SAT * BstarLR - SAB * BstarLL, ih);
-  // branch selectors as 0/1 factors; the reference blends all five candidates with them,
-  // so a non-finite unused candidate still reaches the result (0 * inf = NaN) -- kept.
+  // branch selectors as 0/1 factors; the reference blends all five candidates with them, so
+  // that a non-finite unused candidate reaches the result (0 * inf = NaN). So here, but for the
+  // subsonic one's early exit below.
   const bool Bp = !signbit_of(SB), Tp = !signbit_of(ST), Lp = !signbit_of(SL), Rp = !signbit_of(SR);
   auto on = [](bool b) -> T { return b ? T(1) : T(0); };
   T E = T(0), tmpE;
@@ -499,8 +500,10 @@ __device__ __forceinline__ T emf_z(const Gas<T>& g, const Edge<T>& RT, const Edg
          quot(SAT * SAB, ih) * (AstarT - AstarB) + quot(SAR * SAL, iw) * (BstarR - BstarL);
   const bool middle = !Bp && Tp && !Lp && Rp;
   E += on(middle) * tmpE;
-  // Subsonic in both directions, with a finite candidate: the other four count zero times (they
-  // are finite too: short of overflow their terms are the same products). A wave all of whose
+  // Subsonic in both directions, with a finite candidate: the other four count zero times (a NaN or
+  // infinity among the operands is in this candidate too, through ustar, vstar and the widths; a
+  // product of a speed and a field past the largest double is not, and would have made the blend
+  // NaN, but is outside the range of the quotients, see quot). A wave all of whose
   // lanes are leaves here, without the last fifth of the solve (2D MHD 1024^2 207 -> 204 us per
   // step, 3D MHD 128^3 983 -> 975). Not in FP32, where splitting the solve would change
   // which of its products are fused.

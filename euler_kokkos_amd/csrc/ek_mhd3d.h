@@ -354,7 +354,7 @@ __device__ __forceinline__ void trace_record(const TraceIn<T>& in, const Gas<T>&
 // cells (one wave of 64) and a chunk of planes. Per plane the records of its cells and of
 // the row and column before them go to LDS; then wave t runs task t for the 64 cells: 0 the
 // three Riemann problems, 1..3 the EMF z, y, x. What the plane above needs of this one (the
-// upper z-face state, the two upper edge states of EMF y and x) stays in registers, so only
+// upper z-face state, the two upper edge states of EMF y and x) is kept in LDS beside them, so only
 // one plane of records is ever kept and none goes to memory.
 //
 // Bound by VALU issue and, in the trace, by load latency. With the records in memory (a trace

@@ -27,8 +27,10 @@ extern "C" {
 #define EK_ENOMEM 3   /* device allocation failed */
 
 /* precision of the device state */
-#define EK_FP64 0 /* bit-exact with the reference's CPU results */
-#define EK_FP32 1 /* FP32 state and fluxes, FP64 dt and budgets */
+#define EK_FP64 0 /* bit-exact with the reference's CPU results (densities, pressures and squared fields from
+                   * 1e-60 to 1e60; where products of speeds, densities and fields pass 2.6e269 the step can
+                   * give NaN before the reference's overflows) */
+#define EK_FP32 1 /* FP32 state and fluxes, FP64 dt and budgets (densities below 8.5e37) */
 
 /* host array layouts for ek_upload / ek_download */
 #define EK_LAYOUT_REFERENCE 0 /* Kokkos OpenMP LayoutRight U(i,j[,k],var), ghosts included, FP64 */
