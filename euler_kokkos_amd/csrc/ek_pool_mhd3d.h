@@ -79,8 +79,7 @@ __device__ __forceinline__ void pool_padded_unit(const PoolJobM<T>* __restrict__
 template <class T>
 __global__ __launch_bounds__(256) void mhd3_pool_padprims(const T* __restrict__ Ua, T* __restrict__ W,
                                                           const PoolJobM<T>* __restrict__ jobs,
-                                                          const PoolWork* __restrict__ work, int nwork, TimeSlot* ts,
-                                                          int slot)
+                                                          const PoolWork* __restrict__ work, TimeSlot* ts, int slot)
 {
   pool_padded_unit<T>(jobs, work, ts, slot, [&](const PoolJobM<T>& J, unsigned c) {
     int i, j, k;
@@ -91,8 +90,7 @@ __global__ __launch_bounds__(256) void mhd3_pool_padprims(const T* __restrict__ 
 
 template <class T>
 __global__ __launch_bounds__(256) void mhd3_pool_efield(T* __restrict__ W, const PoolJobM<T>* __restrict__ jobs,
-                                                        const PoolWork* __restrict__ work, int nwork, TimeSlot* ts,
-                                                        int slot)
+                                                        const PoolWork* __restrict__ work, TimeSlot* ts, int slot)
 {
   pool_padded_unit<T>(jobs, work, ts, slot, [&](const PoolJobM<T>& J, unsigned c) {
     int i, j, k;
@@ -193,8 +191,8 @@ inline hipError_t mhd3_launch(const T* Ua, T* Ub, T* W, const PoolJobM<T>* jobs,
 {
   if (np <= 0 || nf <= 0 || nu <= 0)
     return hipSuccess;
-  hipLaunchKernelGGL(mhd3_pool_padprims<T>, dim3(UNITS_P * np), dim3(256), 0, s, Ua, W, jobs, wp, np, ts, slot);
-  hipLaunchKernelGGL(mhd3_pool_efield<T>, dim3(UNITS_P * np), dim3(256), 0, s, W, jobs, wp, np, ts, slot);
+  hipLaunchKernelGGL(mhd3_pool_padprims<T>, dim3(UNITS_P * np), dim3(256), 0, s, Ua, W, jobs, wp, ts, slot);
+  hipLaunchKernelGGL(mhd3_pool_efield<T>, dim3(UNITS_P * np), dim3(256), 0, s, W, jobs, wp, ts, slot);
   hipLaunchKernelGGL((mhd3_pool_fluxemf<T, RS, ST>), dim3(nf), dim3(mhd3::FCN), 0, s, W, jobs, wf, ts, slot);
   hipLaunchKernelGGL(mhd3_pool_update<T>, dim3((unsigned)(ugrid < UNITS_U * nu ? ugrid : UNITS_U * nu)), dim3(256), 0, s,
                      Ua, W, Ub, jobs, wu, nu, ts, slot);
