@@ -14,21 +14,21 @@ pytestmark = pytest.mark.gpu
 ID, IP, IU, IV, IW, IA, IB, IC = range(8)
 
 
-@pytest.mark.parametrize("steps", [1, 4])
-@pytest.mark.parametrize("gamma", ["1.666", "1.4"])
 @pytest.mark.parametrize("rho", [1.0 - 2.0 ** -53, 1.0 - 2.0 ** -52, 4.0 - 2.0 ** -51])
 @pytest.mark.parametrize("mod,ekp", [(test_mhd_gpu, lambda g: test_mhd_gpu.mparams(64, 50, gamma0=g, cfl="0.5")),
                                      (test_mhd3d_gpu, lambda g: test_mhd3d_gpu.m3(20, 18, 16, gamma0=g, cfl="0.5"))],
                          ids=["2d", "3d"])
-def test_root_next_to_a_power_of_two(oracle, mod, ekp, rho, gamma, steps):
-    ekp = ekp(gamma)
-    R0 = np.zeros(oracle.ref_shape(oracle.from_ek(ekp)))
-    rng = np.random.default_rng(7)
-    R0[..., ID] = rho
-    R0[..., IP] = 1.0 / (ekp.gamma0 - 1.0) + 0.375
-    for v in (IA, IB, IC):
-        R0[..., v] = np.where(rng.random(R0.shape[:-1]) < 0.5, 0.5, -0.5)
-    g, o = mod.run_pair(oracle, ekp, R0, steps)
-    print(f"case=field over root rho={rho!r} gamma={gamma} steps={steps}: {np.count_nonzero(g != o)} of {g.size} differ",
-          flush=True)
-    assert np.array_equal(g, o)
+def test_root_next_to_a_power_of_two(oracle, mod, ekp, rho):
+    for gamma in ("1.666", "1.4"):
+        p = ekp(gamma)
+        R0 = np.zeros(oracle.ref_shape(oracle.from_ek(p)))
+        rng = np.random.default_rng(7)
+        R0[..., ID] = rho
+        R0[..., IP] = 1.0 / (p.gamma0 - 1.0) + 0.375
+        for v in (IA, IB, IC):
+            R0[..., v] = np.where(rng.random(R0.shape[:-1]) < 0.5, 0.5, -0.5)
+        for steps in (1, 4):
+            g, o = mod.run_pair(oracle, p, R0, steps)
+            print(f"case=field over root rho={rho!r} gamma={gamma} steps={steps}: {np.count_nonzero(g != o)} of {g.size} differ",
+                  flush=True)
+            assert np.array_equal(g, o)

@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
 ID, IP, IU, IV, IW, IA, IB, IC = range(8)
 PATHS = {"hydro2d": ["hllc", "approx", "llf", "hll"], "hydro3d": ["hllc", "approx", "llf"],
          "mhd2d": ["hlld", "hll", "llf"], "mhd3d": ["hlld", "hll", "llf"]}
+CORNERS = [(1e-60, 1e-60), (1e-60, 1e60), (1e60, 1e-60), (1e60, 1e60), (1e60, 1.0), (1.0, 1e60)]
 
 
 def params(path, riemann):
@@ -48,17 +49,17 @@ def check(oracle, path, ekp, U0, steps, name):
     assert bad == 0
 
 
-@pytest.mark.parametrize("steps", [1, 2])
-@pytest.mark.parametrize("rho,p", [(1e-60, 1e-60), (1e-60, 1e60), (1e60, 1e-60), (1e60, 1e60), (1e60, 1.0), (1.0, 1e60)])
 @pytest.mark.parametrize("path,riemann", [(a, r) for a in PATHS for r in PATHS[a]])
-def test_corners(oracle, path, riemann, rho, p, steps):
-    ekp = params(path, riemann)
-    floors(ekp, rho, p)
-    U0 = test_min_grids_gpu.random_state(oracle, oracle.from_ek(ekp), bool(ekp.mhd), 51)
-    scale = {ID: rho, IP: p, IU: (rho * p) ** 0.5, IV: (rho * p) ** 0.5, IW: (rho * p) ** 0.5}
-    for v in range(U0.shape[-1]):
-        U0[..., v] *= scale.get(v, p ** 0.5)
-    check(oracle, path, ekp, U0, steps, f"{riemann} rho {rho:g} p {p:g}")
+def test_corners(oracle, path, riemann):
+    for rho, p in CORNERS:
+        ekp = params(path, riemann)
+        floors(ekp, rho, p)
+        U0 = test_min_grids_gpu.random_state(oracle, oracle.from_ek(ekp), bool(ekp.mhd), 51)
+        scale = {ID: rho, IP: p, IU: (rho * p) ** 0.5, IV: (rho * p) ** 0.5, IW: (rho * p) ** 0.5}
+        for v in range(U0.shape[-1]):
+            U0[..., v] *= scale.get(v, p ** 0.5)
+        for steps in (1, 2):
+            check(oracle, path, ekp, U0, steps, f"{riemann} rho {rho:g} p {p:g}")
 
 
 @pytest.mark.parametrize("path,riemann", [(a, r) for a in PATHS for r in PATHS[a]])
