@@ -9,9 +9,9 @@ namespace pool {
 
 // 2D tiles the autotuner chooses from (Tile2Of, SmallTile2: ek_hydro.h); the first until tuned.
 // us per step of 24 ragged jobs of up to 320^2, then 100 of up to 512^2 in FP64 / 256 in FP32:
-// FP64 16x12 52.6, 422; 24x8 51.0, 425; small 65.9, 596 (16x16 with 47.6 KB of LDS 58.5, 486).
-// FP32 32x8 29.2, 616; 32x16 29.8, 569; 16x16 28.8, 663; small 41.2, 1010 (16x16 with the loads
-// after the CFL words 29.6, 809). 8 jobs of up to 64^2: small 6.8 and 5.8, the others 7.4 to 7.6.
+// FP64 16x12 47.6, 389; 24x8 44.5, 400; 12x16 44.3, 397; small 61.0, 581. FP32 32x8 29.0, 558;
+// 32x16 27.5, 559; 16x16 26.2, 555; small 38.8, 929. 8 jobs of up to 64^2: small 6.9 and 5.8, the
+// others 7.3 to 7.6.
 struct PoolTile2 {
   int x, y, nt;
   bool cmp;
